@@ -100,6 +100,10 @@ Arena* CurrentArena();
 // in what the arena has left.
 bool WorkspaceFits(size_t bytes);
 
+// Whether a call may ask for this workspace and this temporary now: both fit what the installed
+// arena has left, or exist already, or may grow (no graph capture is running).
+bool ScratchReady(size_t workspace_bytes, TempSlot slot, size_t temp_bytes);
+
 // Stats of include/accel/runtime.h (AcceleratorStats) and the packed-GEMM probes.
 void NoteKernelMatmul();
 // count kernel matmuls at once (a fused caller noting the reference's logical calls).
@@ -345,6 +349,10 @@ struct RmsRequest {
 // stage_b: B may be staged as bf16 parts for the small-grid kernel (StagedF32Parts).
 bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, int64_t m, int64_t k, int64_t n,
                    const Epilogue& epi, hipStream_t stream, const RmsRequest* rms = nullptr, bool stage_b = false);
+// C[m, n] = A[m, k] @ B[k, n] for m <= 16, B fp32 read in place (gemv_f32.hip). False, launching
+// nothing, for sizes it does not take (n < 4, or sides of 2^28 and more).
+bool LaunchGemvF32(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
+                   hipStream_t stream);
 // The int8-weight GEMM on the bf16 matrix cores (exact products, activations split into
 // three bf16 parts): k % 32 == 0, n % 8 == 0, A 16-byte and q 8-byte aligned, per-column or
 // whole-tensor scale, no zero points (a grid of fewer 128 x 128 tiles than CUs splits K).

@@ -221,9 +221,27 @@ void* Workspace(size_t bytes) {
   return ctx.workspace;
 }
 
+namespace {
+void* g_temp[kTempCount] = {};
+size_t g_temp_bytes[kTempCount] = {};
+}  // namespace
+
+bool ScratchReady(size_t workspace_bytes, TempSlot slot, size_t temp_bytes) {
+  if (const Arena* arena = g_arena; arena != nullptr) {
+    const size_t start = (arena->used + 255) & ~size_t(255);
+    const size_t need = ((workspace_bytes + 255) & ~size_t(255)) + temp_bytes;
+    return start <= arena->bytes && need <= arena->bytes - start;
+  }
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if (workspace_bytes <= Ctx().workspace_bytes && temp_bytes <= g_temp_bytes[slot]) return true;
+  }
+  return !Capturing();
+}
+
 void* Temp(TempSlot slot, size_t bytes) {
-  static void* buffers[kTempCount] = {};
-  static size_t sizes[kTempCount] = {};
+  void** buffers = g_temp;
+  size_t* sizes = g_temp_bytes;
   if (void* p = FromArena(bytes, "temporary buffer")) {
     if (slot == kTempArrivals)  // counters must start at zero: cleared by a kernel, not a memset
       LaunchFill(static_cast<float*>(p), 0.f, static_cast<int64_t>((bytes + 3) / 4), Ctx().stream);

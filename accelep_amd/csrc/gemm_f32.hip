@@ -731,6 +731,7 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
   const bool q8 = bq.q != nullptr;
   bool rms_done = false;
   if (q8 && LaunchGemmQ8Bf16(a, bq, c, m, k, n, epi, stream, rms, &rms_done)) return rms_done;
+  if (!q8 && m <= 16 && LaunchGemvF32(a, b, c, m, k, n, epi, stream)) return false;
   const int64_t cus = ctx0.cu_count > 0 ? ctx0.cu_count : 256;
   // Large tiles when they alone give about two workgroups per CU; 64x64 otherwise.
   int bm = 128, bn = 128;
