@@ -2,11 +2,12 @@
 // 0..position+s, head h reads kv head h / (heads / kv_heads), scores = (q . k) / sqrt(head_dim),
 // softmax with the max subtracted, out[d] = sum_t (p_t / sum) * v[t][d].
 //
-// For a prompt (seq > 4), one 512-thread workgroup per (query row, head) holds all of that
-// row's scores in LDS. For a decode step the positions are split over workgroups
-// (AttentionChunkKernel + AttentionCombineKernel below).
+// Fast mode, several rows and head_dim 64 or 128: AttentionFlashKernel, 16 query rows per workgroup on
+// the matrix cores. Otherwise, for a prompt (seq > 4), one 512-thread workgroup per (query row,
+// head) holds all of that row's scores in LDS (AttentionKernel), and for a decode step the
+// positions are split over workgroups (AttentionChunkKernel + AttentionCombineKernel below).
 //
-// Each dot product runs over d in order with separately rounded products, as the
+// In those kernels each dot product runs over d in order with separately rounded products, as the
 // reference does, so scores match it bit for bit; exp, the softmax sums and the weighted
 // sums (interleaved partial sums combined in a fixed order) differ from the reference's
 // sequential loops only by rounding.
@@ -289,196 +290,268 @@ __global__ __launch_bounds__(64) void AttentionCombineKernel(const float* partia
 }
 
 
-// ---- prompt rows, head_dim 64, fast mode: online softmax over key stages ------------------
-// One workgroup per (16 query rows, head), in a 1D grid; its eight waves take an eighth of
-// the keys each and the eighths are combined at the end. Each wave stages 16 keys of K and V
-// in its own LDS slice (coalesced loads; the next stage's loads are issued while the current
-// one is multiplied), so K and V are read once per 16 query rows instead of once per row. The
-// summation order differs from the reference's sequential loops (rounding only), so this
-// path serves the fast mode; the per-row kernel above keeps the reference's score bits.
-constexpr int kFlashRows = 16;
-constexpr int kFlashWaves = 8;
-constexpr int kFlashStage = 16;  // keys per LDS stage
-constexpr int kFlashDim = 64;
-
-constexpr int kFlashStageLoads = kFlashStage * kFlashDim / 4 / 64;  // 16-byte pieces of K (and of V) per lane
-typedef float f4 __attribute__((ext_vector_type(4)));
-
-// Lane l brings float4 (f & 15) of key t0 + (f >> 4), f = i * 64 + l, of K and V; keys past
-// the range read key kend - 1 (masked at use).
-__device__ __forceinline__ void FlashLoadStage(const float* k, const float* v, int64_t t0, int64_t kend,
-                                               int64_t kv_stride, int64_t kv, int lane,
-                                               f4 (&kx)[kFlashStageLoads], f4 (&vx)[kFlashStageLoads]) {
-#pragma unroll
-  for (int i = 0; i < kFlashStageLoads; ++i) {
-    const int f = i * 64 + lane;
-    const int64_t t = min<int64_t>(t0 + (f >> 4), kend - 1);
-    kx[i] = *reinterpret_cast<const f4*>(k + t * kv_stride + kv * kFlashDim + (f & 15) * 4);
-    vx[i] = *reinterpret_cast<const f4*>(v + t * kv_stride + kv * kFlashDim + (f & 15) * 4);
-  }
-}
-
-// Both products run on v_mfma_f32_16x16x4f32. Per stage a wave forms S^T = K Q^T (16 keys x 16
-// rows, 16 MFMAs over the 64 dims) and O^T += V^T P^T (64 dims x 16 rows, 16 MFMAs). Lane l
-// serves row j = l % 16 and key group g = l / 16: the S^T tile leaves it the scores of keys
-// 4g .. 4g + 3 for row j, which is exactly its operand of P^T when the k slot g of step s is
-// key 4g + s, and the O^T tiles hold row j too, so the softmax rescale needs no lane exchange.
-// A row's max and sum meet over the four key groups through two lane swaps.
-constexpr int kMfmaPad = kFlashDim + 4;  // LDS row stride: the 16 key rows fall on distinct banks
+// ---- prompt rows, head_dim 64 or 128, fast mode: online softmax over key stages ----------
+// One workgroup per (16 query rows, head), in a 1D grid; its waves take a part of the keys each
+// and the parts are combined through LDS at the end. The summation order differs from the
+// reference's sequential loops (rounding only), so this path serves the fast mode; the per-row
+// kernel above keeps the reference's score bits.
+//
+// Bound: fp32 MFMA at large sizes (2 * 2 * D flops per visible (row, key) pair), the serial chain
+// of a wave's stages (two MFMA chains and the softmax between them) at small ones. Both products
+// run on v_mfma_f32_16x16x4f32 with every operand straight from memory, no LDS and no barrier in
+// the loop. Lane l serves query row j = l % 16 and group g = l / 16. Per 16 keys a wave forms
+//  * S^T = K Q^T (16 keys x 16 rows): k slot g of step s is dim g * D/4 + s, so a lane's A
+//    operands are D/4 consecutive floats of key row l % 16 and its B operands D/4 consecutive
+//    floats of query row j. The steps alternate between two accumulators, which halves the
+//    chain of dependent MFMAs;
+//  * O^T += V^T P^T: the S^T tile leaves lane l the scores of keys 4g .. 4g + 3 of row j, its own
+//    operand of P^T when k slot g of step s is key 4g + s; the A operand of dim tile (c, t) is
+//    float t of the 16 bytes at V[key 4g + s][64c + 4 (l % 16)], so one 16-byte load feeds four
+//    MFMAs. The O^T tiles hold row j too: the softmax rescale needs no lane exchange.
+// The next stage's keys are requested before the softmax, this stage's values before S^T.
+// Measured, us (workgroup per row and head, all scores in LDS -> here): 512 rows, 9 heads of 64,
+// 94 -> 12.5; 1024 rows, 268 -> 27; 2048 rows, 32 heads, 3119 -> 208 (83 TFLOP/s of the 154 an
+// fp32 matrix product reaches); 1024 rows from position 1500, 16 heads of 128, 4176 -> 190. Four
+// waves: eight took 210 and 204 us of the last two; 32 rows per workgroup 207 and 204, and 18.0
+// of the first; both stages double-buffered 217, 231 and 13.4 (the waits are not the loads').
+constexpr int kFlashWaves = 4;
+constexpr int kFlashThreads = 64 * kFlashWaves;
+constexpr int kFlashRows = 16;  // query rows of a workgroup
+constexpr int kFlashKeys = 16;  // keys a wave takes per step
+constexpr int kFlashPad = 4;
 
 typedef float mv4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(kFlashWaves * 64) void AttentionFlashMfmaKernel(
-    const float* q, const float* k, const float* v, float* out, const int32_t* position_dev, int32_t seq,
-    int32_t position_arg, int32_t heads, int32_t kv_heads) {
-  __shared__ __align__(16) float ks[kFlashWaves][kFlashStage][kMfmaPad];
-  __shared__ __align__(16) float vs[kFlashWaves][kFlashStage][kMfmaPad];
+// A row whose sums are not finite: the masked keys of a stage enter the MFMA as 0 * v, which a
+// non-finite v of a key that the row does not see turns into NaN. The row is formed again here
+// over its visible keys [t0, t1) alone, as AttentionKernel forms it, in chunks of a thread a key.
+// Thread d < dim returns with column d: top the largest score, sum the sum of e^(score - top) and
+// acc that of e^(score - top) * v[t][d].
+struct FlashRow {
+  float top, sum, acc;
+};
+__device__ FlashRow FlashRowAgain(const float* qrow, const float* k, const float* v, int64_t t0, int64_t t1,
+                                  int64_t kv_stride, int dim, float scale, float* es, float* red) {
+  constexpr int kThreads = kFlashThreads;
+  const int tid = threadIdx.x;
+  const auto score = [&](int64_t t) {
+    float dot = 0.f;
+    for (int d = 0; d < dim; ++d) dot = __fadd_rn(dot, __fmul_rn(qrow[d], k[t * kv_stride + d]));
+    return __fmul_rn(dot, scale);
+  };
+  FlashRow row{-INFINITY, 0.f, 0.f};
+  for (int64_t t = t0 + tid; t < t1; t += kThreads) row.top = fmaxf(row.top, score(t));
+  row.top = WaveButterfly(row.top, [](float a, float b) { return fmaxf(a, b); });
+  __syncthreads();
+  if ((tid & 63) == 0) red[tid >> 6] = row.top;
+  __syncthreads();
+  for (int w = 0; w < kThreads / 64; ++w) row.top = fmaxf(row.top, red[w]);
+  for (int64_t c0 = t0; c0 < t1; c0 += kThreads) {
+    const int n = static_cast<int>(min<int64_t>(kThreads, t1 - c0));
+    __syncthreads();
+    if (tid < n) es[tid] = expf(__fsub_rn(score(c0 + tid), row.top));
+    __syncthreads();
+    if (tid < dim) {
+      for (int t = 0; t < n; ++t) {
+        row.sum = __fadd_rn(row.sum, es[t]);
+        row.acc = __fadd_rn(row.acc, __fmul_rn(es[t], v[(c0 + t) * kv_stride + tid]));
+      }
+    }
+  }
+  __syncthreads();
+  return row;
+}
+
+// With splits > 1 the keys of a block are cut into that many ranges, one workgroup each, which
+// leaves its (m, l, acc) of every row in `partial` [seq * heads][splits][2 + D] for
+// AttentionCombineKernel.
+template <int D>
+__global__ __launch_bounds__(kFlashThreads) void AttentionFlashKernel(const float* q, const float* k, const float* v,
+                                                                      float* out, const int32_t* position_dev,
+                                                                      int32_t seq, int32_t position_arg, int32_t heads,
+                                                                      int32_t kv_heads, int32_t splits,
+                                                                      float* partial) {
+  constexpr int kDq = D / 4;  // dims of a lane's S^T operands
+  constexpr int kC = D / 64;  // 16-byte pieces of a value row per lane
+  __shared__ __align__(16) float part_o[kFlashWaves][kFlashRows][D + kFlashPad];
   __shared__ float part_m[kFlashWaves][kFlashRows];
   __shared__ float part_l[kFlashWaves][kFlashRows];
+  __shared__ uint32_t again;  // rows of the block to form again
   const int64_t position = position_dev != nullptr ? *position_dev : position_arg;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int j = lane & 15;  // query row of the block
-  const int g = lane >> 4;  // key group / dim group
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15;
+  const int g = lane >> 4;
   // Heaviest row blocks first, over all heads: the workgroups beyond one per CU are then the
   // blocks with the fewest keys, and no two long blocks share a CU.
-  const int32_t unit = static_cast<int32_t>(blockIdx.x);
-  const int32_t qblocks = static_cast<int32_t>(gridDim.x) / heads;
+  const int32_t split = static_cast<int32_t>(blockIdx.x) % splits;
+  const int32_t unit = static_cast<int32_t>(blockIdx.x) / splits;
+  const int32_t qblocks = static_cast<int32_t>(gridDim.x) / (heads * splits);
   const int32_t rank = unit / heads;
   const int64_t s0 = static_cast<int64_t>(qblocks - 1 - rank) * kFlashRows;
   const int64_t h = unit - rank * heads;
   const int64_t kv = h / (heads / kv_heads);
-  const int64_t row = s0 + j;
-  const bool live = row < seq;
-  const int64_t last_key = position + (live ? row : -1);  // keys 0 .. last_key (causal)
-  const float scale = __fdiv_rn(1.f, __fsqrt_rn(static_cast<float>(kFlashDim)));
+  const int64_t kv_stride = static_cast<int64_t>(kv_heads) * D;
+  const float scale = __fdiv_rn(1.f, __fsqrt_rn(static_cast<float>(D)));
+  const float* kh = k + kv * D;
+  const float* vh = v + kv * D;
 
-  // B operand of S^T: q[row j][16 g + s], s = 0 .. 15.
-  float qb[16];
+  const int64_t row_j = s0 + j;
+  const int64_t last_key = row_j < seq ? position + row_j : -1;  // row j sees keys 0 .. last_key (causal)
+  mv4 qb[kDq / 4];
   {
-    const float* qrow = q + ((live ? row : 0) * heads + h) * kFlashDim + 16 * g;
+    const mv4* src = reinterpret_cast<const mv4*>(q + ((row_j < seq ? row_j : seq - 1) * heads + h) * D + kDq * g);
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      const float4 x = *reinterpret_cast<const float4*>(qrow + i);
-      qb[i] = x.x;
-      qb[i + 1] = x.y;
-      qb[i + 2] = x.z;
-      qb[i + 3] = x.w;
-    }
+    for (int i = 0; i < kDq / 4; ++i) qb[i] = src[i];
   }
   const int64_t nkeys = position + min<int64_t>(s0 + kFlashRows, seq);
-  const int64_t per = ((nkeys + kFlashWaves - 1) / kFlashWaves + kFlashStage - 1) / kFlashStage * kFlashStage;
-  const int64_t kbeg = min<int64_t>(wave * per, nkeys);
-  const int64_t kend = min<int64_t>(kbeg + per, nkeys);
-  const int64_t kv_stride = kv_heads * kFlashDim;
+  const int64_t parts = static_cast<int64_t>(splits) * kFlashWaves;
+  const int64_t per = ((nkeys + parts - 1) / parts + kFlashKeys - 1) / kFlashKeys * kFlashKeys;
+  const int64_t wg_beg = min<int64_t>(split * kFlashWaves * per, nkeys);  // the workgroup's keys
+  const int64_t wg_end = min<int64_t>(wg_beg + kFlashWaves * per, nkeys);
+  const int64_t kbeg = min<int64_t>(wg_beg + wave * per, wg_end);
+  const int64_t kend = min<int64_t>(kbeg + per, wg_end);
+  // Keys past the wave's range read its last key (masked at use).
+  mv4 kx[kDq / 4], vx[4][kC];
+  const auto load_k = [&](int64_t t0) {
+    const mv4* src = reinterpret_cast<const mv4*>(kh + min<int64_t>(t0 + j, kend - 1) * kv_stride + kDq * g);
+#pragma unroll
+    for (int i = 0; i < kDq / 4; ++i) kx[i] = src[i];
+  };
+  const auto load_v = [&](int64_t t0) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const mv4* src = reinterpret_cast<const mv4*>(vh + min<int64_t>(t0 + 4 * g + s, kend - 1) * kv_stride + 4 * j);
+#pragma unroll
+      for (int c = 0; c < kC; ++c) vx[s][c] = src[16 * c];
+    }
+  };
 
   float m = -INFINITY;
   float l = 0.f;  // this lane's share (its key groups) of row j's sum
-  mv4 acc_o[4];
+  mv4 acc_o[kC][4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc_o[t] = mv4{0.f, 0.f, 0.f, 0.f};
-
-  f4 kx[kFlashStageLoads], vx[kFlashStageLoads];
-  if (kbeg < kend) FlashLoadStage(k, v, kbeg, kend, kv_stride, kv, lane, kx, vx);
-  for (int64_t t0 = kbeg; t0 < kend; t0 += kFlashStage) {  // uniform across the wave
+  for (int c = 0; c < kC; ++c)
 #pragma unroll
-    for (int i = 0; i < kFlashStageLoads; ++i) {
-      const int f = i * 64 + lane;
-      *reinterpret_cast<f4*>(&ks[wave][f >> 4][(f & 15) * 4]) = kx[i];
-      *reinterpret_cast<f4*>(&vs[wave][f >> 4][(f & 15) * 4]) = vx[i];
-    }
-    if (t0 + kFlashStage < kend) FlashLoadStage(k, v, t0 + kFlashStage, kend, kv_stride, kv, lane, kx, vx);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // S^T[key i][row j]: A = K[key l % 16][16 g + s], B = q[row][16 g + s].
-    float kr[16];
+    for (int t = 0; t < 4; ++t) acc_o[c][t] = mv4{0.f, 0.f, 0.f, 0.f};
+  if (kbeg < kend) load_k(kbeg);
+  for (int64_t t0 = kbeg; t0 < kend; t0 += kFlashKeys) {  // uniform across the wave
+    load_v(t0);
+    __builtin_amdgcn_sched_barrier(0);
+    mv4 st0 = mv4{0.f, 0.f, 0.f, 0.f}, st1 = st0;
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      const float4 x = *reinterpret_cast<const float4*>(&ks[wave][j][16 * g + i]);
-      kr[i] = x.x;
-      kr[i + 1] = x.y;
-      kr[i + 2] = x.z;
-      kr[i + 3] = x.w;
-    }
-    mv4 st = mv4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < kDq / 4; ++i)
 #pragma unroll
-    for (int s = 0; s < 16; ++s) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[s], qb[s], st, 0, 0, 0);
+      for (int e = 0; e < 4; e += 2) {
+        st0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[i][e], qb[i][e], st0, 0, 0, 0);
+        st1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[i][e + 1], qb[i][e + 1], st1, 0, 0, 0);
+      }
+    const mv4 st = st0 + st1;
+    if (t0 + kFlashKeys < kend) load_k(t0 + kFlashKeys);
+    __builtin_amdgcn_sched_barrier(0);
     // Lane (j, g) holds the scores of keys t0 + 4 g + r, r = 0 .. 3, for row j.
-    float sc[4];
+    const int64_t seen = min<int64_t>(kend - 1, last_key);
+    float p[4];
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int64_t t = t0 + 4 * g + r;
-      sc[r] = (t < kend && t <= last_key) ? __fmul_rn(st[r], scale) : -INFINITY;
-      mx = fmaxf(mx, sc[r]);
+      p[r] = t0 + 4 * g + r <= seen ? __fmul_rn(st[r], scale) : -INFINITY;
+      mx = fmaxf(mx, p[r]);
     }
     mx = fmaxf(mx, XorLane<16>(mx));
     mx = fmaxf(mx, XorLane<32>(mx));
     const float m_new = fmaxf(m, mx);
     const bool none = m_new == -INFINITY;  // nothing of this row so far
-    const float corr = (m == -INFINITY || none) ? (none ? 1.f : 0.f) : expf(m - m_new);
-    float pr[4];
+    const float corr = m == -INFINITY ? (none ? 1.f : 0.f) : expf(m - m_new);
     float psum = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      pr[r] = sc[r] == -INFINITY ? 0.f : expf(sc[r] - m_new);
-      psum = psum + pr[r];
+      p[r] = p[r] == -INFINITY ? 0.f : expf(p[r] - m_new);
+      psum = psum + p[r];
     }
     l = l * corr + psum;
-    m = none ? m : m_new;
+    m = m_new;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc_o[t] = acc_o[t] * corr;
-    // O^T[dim 16 t + i][row j] += V^T[dim][key 4 g + s] P^T[key 4 g + s][row j].
+    for (int c = 0; c < kC; ++c)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc_o[c][t] = acc_o[c][t] * corr;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        acc_o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[wave][4 * g + s][16 * t + j], pr[s], acc_o[t], 0, 0, 0);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the stage is read before the next one overwrites it
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int c = 0; c < kC; ++c)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc_o[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[s][c][t], p[s], acc_o[c][t], 0, 0, 0);
   }
-  // Row j's sum over the four key groups; then the waves' eighths meet in LDS. acc_o[t][r] is
-  // O^T[dim 16 t + 4 g + r][row j]; the wave's stage rows hold its 16 x 64 block.
+  // Row j's sum over the four key groups; then the waves' parts meet in LDS. acc_o[c][t][r] is
+  // O^T[dim 64c + 16g + 4r + t][row j].
   l = l + XorLane<16>(l);
   l = l + XorLane<32>(l);
-  float* part_acc = &ks[wave][0][0];  // [16 rows][kMfmaPad]: this wave's stage, no longer read
   if (g == 0) {
     part_m[wave][j] = m;
     part_l[wave][j] = l;
   }
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-    *reinterpret_cast<float4*>(&part_acc[j * kMfmaPad + 16 * t + 4 * g]) =
-        make_float4(acc_o[t][0], acc_o[t][1], acc_o[t][2], acc_o[t][3]);
-  __syncthreads();
-  if (wave == 0 && live) {
-    float big = part_m[0][j];
+  for (int c = 0; c < kC; ++c)
 #pragma unroll
-    for (int w = 1; w < kFlashWaves; ++w) big = fmaxf(big, part_m[w][j]);
-    float wts[kFlashWaves];
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<mv4*>(&part_o[wave][j][64 * c + 16 * g + 4 * r]) =
+          mv4{acc_o[c][0][r], acc_o[c][1][r], acc_o[c][2][r], acc_o[c][3][r]};
+  if (tid == 0) again = 0;
+  __syncthreads();
+  for (int item = tid; item < kFlashRows * kDq; item += kFlashThreads) {
+    const int rl = item / kDq;
+    const int d4 = item % kDq;
+    const int64_t row = s0 + rl;
+    if (row >= seq) continue;
+    float big = part_m[0][rl];
+#pragma unroll
+    for (int w = 1; w < kFlashWaves; ++w) big = fmaxf(big, part_m[w][rl]);
     float total = 0.f;
+    mv4 o = mv4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < kFlashWaves; ++w) {
-      wts[w] = part_m[w][j] == -INFINITY ? 0.f : expf(part_m[w][j] - big);
-      total = total + wts[w] * part_l[w][j];
+      const float mw = part_m[w][rl];
+      const float wt = mw == -INFINITY ? 0.f : expf(mw - big);
+      total = total + wt * part_l[w][rl];
+      o = o + wt * *reinterpret_cast<const mv4*>(&part_o[w][rl][4 * d4]);
     }
-    float* orow = out + (row * heads + h) * kFlashDim;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float o[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < kFlashWaves; ++w) {
-        const float4 x = *reinterpret_cast<const float4*>(&ks[w][0][0] + j * kMfmaPad + 16 * t + 4 * g);
-        o[0] = o[0] + wts[w] * x.x;
-        o[1] = o[1] + wts[w] * x.y;
-        o[2] = o[2] + wts[w] * x.z;
-        o[3] = o[3] + wts[w] * x.w;
+    if (splits > 1) {
+      float* dst = partial + ((row * heads + h) * splits + split) * (2 + D);
+      if (d4 == 0) {
+        dst[0] = big;
+        dst[1] = total;
       }
-      *reinterpret_cast<float4*>(orow + 16 * t + 4 * g) =
-          make_float4(o[0] / total, o[1] / total, o[2] / total, o[3] / total);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dst[2 + 4 * d4 + e] = o[e];
+    } else {
+      o = mv4{__fdiv_rn(o[0], total), __fdiv_rn(o[1], total), __fdiv_rn(o[2], total), __fdiv_rn(o[3], total)};
+      *reinterpret_cast<mv4*>(out + (row * heads + h) * D + 4 * d4) = o;
+    }
+    // inf - inf and NaN - NaN are NaN: any other difference of a value and itself is 0.
+    if (o[0] - o[0] != 0.f || o[1] - o[1] != 0.f || o[2] - o[2] != 0.f || o[3] - o[3] != 0.f)
+      atomicOr(&again, 1u << rl);
+  }
+  __syncthreads();
+  const uint32_t redo = again;
+  if (redo == 0) return;  // uniform
+  for (int rl = 0; rl < kFlashRows; ++rl) {
+    if ((redo >> rl & 1u) == 0) continue;
+    const int64_t row = s0 + rl;
+    const int64_t seen = min<int64_t>(wg_end, position + row + 1);
+    const FlashRow x = FlashRowAgain(q + (row * heads + h) * D, kh, vh, wg_beg, seen, kv_stride, D, scale,
+                                     &part_o[0][0][0], &part_m[0][0]);
+    if (tid >= D) continue;
+    if (splits > 1) {
+      float* dst = partial + ((row * heads + h) * splits + split) * (2 + D);
+      dst[2 + tid] = x.acc;
+      if (tid == 0) {
+        dst[0] = x.top;
+        dst[1] = x.sum;
+      }
+    } else {
+      out[(row * heads + h) * D + tid] = __fdiv_rn(x.acc, x.sum);
     }
   }
 }
@@ -896,6 +969,45 @@ size_t AttentionWorkBytes(int64_t seq, int64_t heads, int64_t max_position, int6
   return 0;
 }
 
+namespace {
+
+int64_t CuCount() {
+  const Context& ctx = Ctx();
+  return ctx.cu_count > 0 ? ctx.cu_count : 256;
+}
+
+void LaunchFlash(const float* q, const float* k, const float* v, float* out, int64_t seq, int64_t position,
+                 int64_t heads, int64_t kv_heads, int64_t head_dim, hipStream_t stream, const int32_t* position_dev,
+                 int64_t top) {
+  const int64_t blocks = (seq + kFlashRows - 1) / kFlashRows * heads;
+  if (heads > 65535 || seq > 0x7fffffff || position > 0x7fffffff || kv_heads > 65535 || blocks > 0x7fffffff)
+    Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention is too large");
+  const int64_t cus = CuCount();
+  // A grid that leaves CUs idle over a long key range cuts the range, at least 128 keys each (the
+  // combine costs about 3 us): 17 rows from position 500, 9 heads, 12.0 -> 9.5 us in four; 100 rows
+  // from 1700, 4 heads of 128, 52 -> 16 us in eight; 300 rows from 0, 4 heads, 13.9 -> 14.4 in two.
+  int64_t splits = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, (top + seq) / 128));
+  const size_t bytes = static_cast<size_t>(seq * heads * splits * (2 + head_dim)) * sizeof(float);
+  if (splits > 1 && !ScratchReady(bytes, kTempFlags, 0)) splits = 1;
+  float* partial = splits > 1 ? static_cast<float*>(Workspace(bytes)) : nullptr;
+  const dim3 grid(static_cast<uint32_t>(blocks * splits)), block(kFlashThreads);
+#define ACCEL_FLASH(D)                                                                                            \
+  hipLaunchKernelGGL(AttentionFlashKernel<D>, grid, block, 0, stream, q, k, v, out, position_dev,                 \
+                     static_cast<int32_t>(seq), static_cast<int32_t>(position), static_cast<int32_t>(heads), \
+                     static_cast<int32_t>(kv_heads), static_cast<int32_t>(splits), partial)
+  if (head_dim == 64) ACCEL_FLASH(64);
+  else ACCEL_FLASH(128);
+#undef ACCEL_FLASH
+  Check(hipGetLastError(), "AttentionFlashKernel launch");
+  if (splits > 1) {
+    hipLaunchKernelGGL(AttentionCombineKernel, dim3(static_cast<uint32_t>(seq * heads)), dim3(64), 0, stream, partial, out,
+                       splits, head_dim);
+    Check(hipGetLastError(), "AttentionCombineKernel launch");
+  }
+}
+
+}  // namespace
+
 void LaunchAttention(const float* q, const float* k, const float* v, float* out, int64_t seq, int64_t position,
                      int64_t heads, int64_t kv_heads, int64_t head_dim, hipStream_t stream, const int32_t* position_dev,
                      int64_t max_position, float* work, size_t work_bytes, bool fast) {
@@ -919,6 +1031,15 @@ void LaunchAttention(const float* q, const float* k, const float* v, float* out,
   const bool aligned = (reinterpret_cast<uintptr_t>(k) % 16 == 0) && (reinterpret_cast<uintptr_t>(v) % 16 == 0) &&
                        head_dim % 4 == 0;
   const int vec = aligned ? static_cast<int>(head_dim) : 0;
+  // Two to four rows over a long key range go to the flash kernel only where one workgroup per
+  // (row, head, 64 positions) would come to several per CU (3 rows from position 8000, 32 heads:
+  // 109 -> 36 us, 4 from 1775, 9 heads of 128: 17.5 -> 14.8; 2 from 1775, 9 heads: 9.2 -> 10.3).
+  const bool few = seq <= kSplitMaxSeq && rows >= 256 && blocks * ((rows + kChunk - 1) / kChunk) < 3 * CuCount();
+  if (fast && seq > 1 && !few && (head_dim == 64 || head_dim == 128) && aligned && (reinterpret_cast<uintptr_t>(q) % 16 == 0) &&
+      (reinterpret_cast<uintptr_t>(out) % 16 == 0)) {
+    LaunchFlash(q, k, v, out, seq, position, heads, kv_heads, head_dim, stream, position_dev, top);
+    return;
+  }
   if (seq <= kSplitMaxSeq) {
     const int64_t chunks = (rows + kChunk - 1) / kChunk;
     if (chunks > kMaxChunks) Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention context is too long for a decode step");
@@ -938,18 +1059,6 @@ void LaunchAttention(const float* q, const float* k, const float* v, float* out,
     hipLaunchKernelGGL(AttentionCombineKernel, dim3(static_cast<uint32_t>(blocks)), dim3(64), 0, stream, scratch, out,
                        chunks, head_dim);
     Check(hipGetLastError(), "AttentionCombineKernel launch");
-    return;
-  }
-  if (fast && head_dim == kFlashDim && aligned && (reinterpret_cast<uintptr_t>(q) % 16 == 0) &&
-      (reinterpret_cast<uintptr_t>(out) % 16 == 0)) {
-    const int64_t qblocks = (seq + kFlashRows - 1) / kFlashRows;
-    if (qblocks > 0x7fffffff || heads > 65535 || seq > 0x7fffffff || position > 0x7fffffff || kv_heads > 65535)
-      Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention is too large");
-    if (qblocks * heads > 0x7fffffff) Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention is too large");
-    hipLaunchKernelGGL(AttentionFlashMfmaKernel, dim3(static_cast<uint32_t>(qblocks * heads)),
-                       dim3(kFlashWaves * 64), 0, stream, q, k, v, out, position_dev, static_cast<int32_t>(seq),
-                       static_cast<int32_t>(position), static_cast<int32_t>(heads), static_cast<int32_t>(kv_heads));
-    Check(hipGetLastError(), "AttentionFlashMfmaKernel launch");
     return;
   }
   float* spill = rows > kLdsScores ? scratch : nullptr;

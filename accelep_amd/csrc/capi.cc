@@ -431,7 +431,7 @@ ACCEL_HIP_API int accel_hip_attention(AccelHipBuffer q, AccelHipBuffer k, AccelH
     NoteDeviceWrite(out.data, CheckedFloats(seq, heads, head_dim));
     LaunchAttention(static_cast<const float*>(q.data), static_cast<const float*>(k.data),
                     static_cast<const float*>(v.data), static_cast<float*>(out.data), seq, position, heads, kv_heads,
-                    head_dim, Ctx().stream);
+                    head_dim, Ctx().stream, nullptr, 0, nullptr, 0, !Ctx().exact_products);
   });
 }
 

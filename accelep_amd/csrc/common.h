@@ -399,7 +399,7 @@ void LaunchAdvance(int32_t* state, hipStream_t stream);
 // max_position: with position_dev, the largest position the device word may hold. work /
 // work_bytes: caller-owned scratch (at least AttentionWorkBytes); null uses the library
 // workspace.
-// fast: prompt rows (seq > 4) with head_dim 64 may use the online-softmax kernel, whose sums
+// fast: several rows (seq > 1) with head_dim 64 or 128 may use the online-softmax kernel, whose sums
 // run in another order than the reference's (rounding only); otherwise the scores keep the
 // reference's bits.
 void LaunchAttention(const float* q, const float* k, const float* v, float* out, int64_t seq, int64_t position,

@@ -208,7 +208,9 @@ ACCEL_HIP_API int accel_hip_rope(AccelHipBuffer states, AccelHipBuffer cos_table
 ACCEL_HIP_API int accel_hip_append_cache(AccelHipBuffer src, AccelHipBuffer cache, int64_t seq, int64_t position,
                                          int64_t n_heads, int64_t head_dim);
 /* Device::Attention (device.h:110-112; src/sim_attend.cc:9-46). scores is not used as
- * scratch by the HIP kernel but must still be large enough, as in the reference. */
+ * scratch by the HIP kernel but must still be large enough, as in the reference. Several rows
+ * (seq > 1) with head_dim 64 or 128 form their scores and sums on the fp32 matrix cores in another
+ * order than the reference's (rounding only) unless exact products are on. */
 ACCEL_HIP_API int accel_hip_attention(AccelHipBuffer q, AccelHipBuffer k, AccelHipBuffer v, AccelHipBuffer scores,
                                       AccelHipBuffer out, int64_t seq, int64_t position, int64_t heads,
                                       int64_t kv_heads, int64_t head_dim);
