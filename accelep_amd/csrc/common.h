@@ -354,8 +354,9 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
 bool LaunchGemvF32(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
                    hipStream_t stream);
 // The int8-weight GEMM on the bf16 matrix cores (exact products, activations split into
-// three bf16 parts): k % 32 == 0, n % 8 == 0, A 16-byte and q 8-byte aligned, per-column or
-// whole-tensor scale, no zero points (a grid of fewer 128 x 128 tiles than CUs splits K).
+// three bf16 parts): k >= 32, n >= 8 (a grid that leaves CUs idle splits K where the workspace
+// for it can be had). The staged-copy kernels take k % 32 == 0, n % 8 == 0, A 16-byte and q 8-byte
+// aligned, per-column or whole-tensor scale, no zero points.
 // With b.bf16 (GemmWantsBf16Image) the activations are split once per call into an image
 // the tiles copy as-is, the weight operands come from the staged bf16 copy, and an rms
 // request is served inside (per-tile row sums of squares, then one scaling pass); *rms_done

@@ -1,6 +1,6 @@
 // fp32 GEMM on the matrix cores: C[m, n] = A[m, k] @ B[k, n] (+ fused epilogue), B either
 // fp32 (Device::MatMul, src/sim_device.cc:185-196) or an int8 plane dequantized panel by
-// panel into LDS (accel::MatMulQuantized for m > 16, src/sim_device.cc:541-602).
+// panel into LDS (accel::MatMulQuantized for m > 16 with k < 32 or n < 8, src/sim_device.cc:541-602).
 //
 // Bound: MFMA (fp32, v_mfma_f32_32x32x2_f32). 2*m*n*k flops per call.
 //

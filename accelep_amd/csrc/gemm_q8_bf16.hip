@@ -1,6 +1,6 @@
 // int8-weight GEMM on the bf16 matrix cores: C[m, n] = A[m, k] @ (q[k, n] * scale) for
-// accel::MatMulQuantized with m > 16 (src/sim_device.cc:541-602), per-column or whole-tensor
-// scale, no zero points.
+// accel::MatMulQuantized with m > 16 (src/sim_device.cc:541-602), any scale and zero points (the
+// staged-copy kernels further down: per-column or whole-tensor scale, no zero points).
 //
 // Exact products on v_mfma_f32_32x32x16_bf16:
 //  * every weight byte is an integer in [-128, 127], which bf16 holds exactly;
@@ -28,8 +28,15 @@
 //    per chunk.
 //  * Tiles are dealt to the 8 XCDs in contiguous runs, ordered in bands of 4 row tiles, so
 //    the workgroups resident on one XCD share A rows and W columns in its L2.
-//  * A grid of fewer tiles than CUs splits K (whole chunks); the partial sums go to the
+//  * A grid that leaves CUs idle splits K (whole chunks, PlanQ8Gemm); the partial sums go to the
 //    workspace and SplitReduceKernel adds them in split order, scales and applies the epilogue.
+//  * Zero points, a per-row scale, a k of no whole chunks, an n of no whole octets and unaligned
+//    operands take the same kernel in its general forms (Form below): the conversions of the W
+//    panel gain a subtraction, a ragged k zeroes part of its first chunk, loads need no alignment.
+//    They had run on the fp32 matrix cores with each panel dequantized on the way into LDS:
+//    333 x 4096 x 4096 with zero points 223 us (50 TFLOP/s) -> 55, with a per-row scale 227 -> 56,
+//    333 x 4095 x 4097 440 -> 62, 2000 x 2047 x 14335 1651 -> 405, 2000 x 2048 x 14336 with zero
+//    points 1011 -> 383. Error against float64 at k = 4096: 1.1e-6 -> 1.1e-7 .. 2.5e-7.
 #include "device_common.h"
 
 #include <algorithm>
@@ -65,58 +72,118 @@ struct Q8GemmArgs {
   const float* a;
   const int8_t* q;
   const float* scale;
+  const int8_t* zero;  // nullptr: zero points 0
   int32_t mode;
   int64_t const_index;
   float* c;
   int64_t m, k, n;
   int32_t tiles_m, tiles_n, tiles, tiles_per_xcd;
-  int64_t k_per_split;  // a multiple of kBK
-  float* partials;      // [splits][m][n] raw sums when the K range is split, else nullptr
+  int64_t chunks_per_split;
+  float* partials;  // [splits][m][n] raw sums when the K range is split, else nullptr
   Epilogue epi;
 };
+
+// What a launch's operands look like. kPlain: whole chunks and octets, aligned, no zero points,
+// per-column or whole-tensor scale. The others take any k >= 32, n >= 8 and alignment: kCols with
+// per-column (or whole-tensor) zero points or none, kRows with a per-row scale (and zero points).
+// There q - z is an integer in [-255, 255], which bf16 holds exactly, and a per-row scale
+// multiplies A (fl(x * s), one rounding where the reference rounds (q - z) * s).
+enum Form : int { kPlain = 0, kCols = 1, kRows = 2 };
+
+// First k of chunk ch. A ragged k puts its short chunk first: chunk 0 reads k 0 .. 31 and keeps
+// the first 32 - pad of them, the later ones are whole, so only the prologue masks.
+template <int kForm>
+__device__ __forceinline__ int64_t ChunkK(int64_t ch, int pad) {
+  if constexpr (kForm == kPlain) return ch * kBK;
+  return ch == 0 ? 0 : ch * kBK - pad;
+}
 
 // The global part of one chunk, as loaded: A rows (tid / 8) + 32i, k quad tid % 8; W rows
 // 2 * kp and 2 * kp + 1 of column octet oct, kp = tid / octets < 16 (for BM = 64 the upper
 // half of the threads load no W).
-template <int BM>
+template <int BM, int kForm>
 struct Panels {
-  float4 a[Tile<BM>::kARows];
+  v4f a[Tile<BM>::kARows];
   u32x2 b[2];
+  v4f row_scale;      // kRows: of the thread's k quad
+  float row_zero[2];  // kRows: of its two W rows
 };
 
+// A vector load from an address aligned to its elements only.
+template <typename T>
+__device__ __forceinline__ T LoadAny(const void* src) {
+  T v;
+  __builtin_memcpy(&v, src, sizeof(T));
+  return v;
+}
+
 // Rows and columns past the matrix read a clamped, valid element; their results are never
-// stored (every chunk lies inside k, which is a multiple of kBK).
-template <int BM>
+// stored (every chunk lies inside k).
+template <int BM, int kForm>
 __device__ __forceinline__ void LoadPanels(const Q8GemmArgs& p, int64_t m0, int64_t n0, int64_t k0, int tid,
-                                           Panels<BM>& r) {
+                                           Panels<BM, kForm>& r) {
   const int kq = tid & 7;
 #pragma unroll
   for (int i = 0; i < Tile<BM>::kARows; ++i) {
     const int64_t row = m0 + (tid >> 3) + 32 * i;
     const int64_t rc = row < p.m ? row : p.m - 1;
-    r.a[i] = *reinterpret_cast<const float4*>(p.a + rc * p.k + k0 + 4 * kq);
+    const float* src = p.a + rc * p.k + k0 + 4 * kq;
+    if constexpr (kForm == kPlain) r.a[i] = *reinterpret_cast<const v4f*>(src);
+    else r.a[i] = LoadAny<v4f>(src);
   }
+  if constexpr (kForm == kRows) r.row_scale = LoadAny<v4f>(p.scale + k0 + 4 * kq);
   constexpr int kOcts = Tile<BM>::kOcts;
   const int kp = tid / kOcts;
   if (kp >= kBK / 2) return;
   const int64_t col = n0 + 8 * (tid % kOcts);
-  const int64_t cc = col < p.n ? col : p.n - 8;
+  const int64_t cc = min(col, p.n - 8);
   const int64_t kr = k0 + 2 * kp;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) r.b[h] = *reinterpret_cast<const u32x2*>(p.q + (kr + h) * p.n + cc);
+  for (int h = 0; h < 2; ++h) {
+    const int8_t* src = p.q + (kr + h) * p.n + cc;
+    if constexpr (kForm == kPlain) r.b[h] = *reinterpret_cast<const u32x2*>(src);
+    else r.b[h] = LoadAny<u32x2>(src);
+    if constexpr (kForm == kRows) r.row_zero[h] = p.zero != nullptr ? static_cast<float>(p.zero[kr + h]) : 0.f;
+  }
+}
+
+// A thread's constants of the general forms: how far its octet was moved back to stay inside a
+// row (bits), and the zero points of its columns in the rotated order of StorePanels.
+struct ColConst {
+  int shift;
+  float zero[8];
+};
+
+template <int BM, int kForm>
+__device__ __forceinline__ void LoadColConst(const Q8GemmArgs& p, int64_t n0, int tid, ColConst& cc) {
+  if constexpr (kForm == kPlain) return;
+  const int oct = tid % Tile<BM>::kOcts;
+  const int64_t col = n0 + 8 * oct;
+  cc.shift = 8 * static_cast<int>(min(col - min(col, p.n - 8), int64_t(7)));
+  if constexpr (kForm == kCols) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int64_t gc = min(col + ((c + oct) & 7), p.n - 1);
+      cc.zero[c] = p.zero != nullptr ? static_cast<float>(p.zero[p.mode == kScalePerCol ? gc : p.const_index]) : 0.f;
+    }
+  }
 }
 
 // Word offset of 16-byte k group g (0..3) of LDS row `row`.
 __device__ __forceinline__ int GroupWord(int row, int g) { return row * kRowWords + 4 * (g ^ ((row >> 1) & 3)); }
 
-template <int BM>
-__device__ __forceinline__ void StorePanels(uint32_t* buf, int tid, const Panels<BM>& r) {
+template <int BM, int kForm>
+__device__ __forceinline__ void StorePanels(uint32_t* buf, int tid, const Panels<BM, kForm>& r, const ColConst& cc) {
   constexpr int kAPlaneWords = Tile<BM>::kAPlaneWords;
   const int kq = tid & 7;
 #pragma unroll
   for (int i = 0; i < Tile<BM>::kARows; ++i) {
     const int row = (tid >> 3) + 32 * i;
-    const float x[4] = {r.a[i].x, r.a[i].y, r.a[i].z, r.a[i].w};
+    float x[4] = {r.a[i].x, r.a[i].y, r.a[i].z, r.a[i].w};
+    if constexpr (kForm == kRows) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = __fmul_rn(x[t], r.row_scale[t]);
+    }
     uint32_t part[3][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -143,8 +210,11 @@ __device__ __forceinline__ void StorePanels(uint32_t* buf, int tid, const Panels
   uint32_t rot[2][2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const uint32_t lo = (s & 4) ? r.b[h][1] : r.b[h][0];
-    const uint32_t hi = (s & 4) ? r.b[h][0] : r.b[h][1];
+    u32x2 w = r.b[h];
+    if constexpr (kForm != kPlain)
+      w = __builtin_bit_cast(u32x2, __builtin_bit_cast(uint64_t, w) >> cc.shift);
+    const uint32_t lo = (s & 4) ? w[1] : w[0];
+    const uint32_t hi = (s & 4) ? w[0] : w[1];
     rot[h][0] = __builtin_amdgcn_alignbyte(hi, lo, s & 3);
     rot[h][1] = __builtin_amdgcn_alignbyte(lo, hi, s & 3);
   }
@@ -152,8 +222,15 @@ __device__ __forceinline__ void StorePanels(uint32_t* buf, int tid, const Panels
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     const int nl = 8 * oct + ((c + s) & 7);
-    wplane[GroupWord(nl, kp >> 2) + wsub] =
-        PackBf16(ByteToFloat(rot[0][c >> 2], c & 3), ByteToFloat(rot[1][c >> 2], c & 3));
+    float w0 = ByteToFloat(rot[0][c >> 2], c & 3), w1 = ByteToFloat(rot[1][c >> 2], c & 3);
+    if constexpr (kForm == kCols) {
+      w0 -= cc.zero[c];
+      w1 -= cc.zero[c];
+    } else if constexpr (kForm == kRows) {
+      w0 -= r.row_zero[0];
+      w1 -= r.row_zero[1];
+    }
+    wplane[GroupWord(nl, kp >> 2) + wsub] = PackBf16(w0, w1);
   }
 }
 
@@ -192,7 +269,70 @@ __device__ __forceinline__ void ComputeChunk(const uint32_t* buf, int lane, int 
   }
 }
 
+// The wave's raw sums over k [kb, ke) on v_mfma_f32_32x32x2f32 with both operands straight from
+// memory: for tiles whose values the bf16 parts cannot hold (infinities, NaN, the last binade
+// below the fp32 limit, or values so small that the parts leave the normal range). Slow (a dword
+// load per operand), and only such tiles take it.
 template <int BM>
+__device__ void PlainSums(const Q8GemmArgs& p, int64_t m0, int64_t n0, int64_t kb, int64_t ke, int lane, int wm, int wn,
+                          v16f (&acc)[Tile<BM>::kS][Tile<BM>::kS]) {
+  constexpr int S = Tile<BM>::kS;
+  const float* arow[S];
+  int64_t col[S];
+  float zc[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    arow[i] = p.a + min(m0 + wm * (BM / 2) + i * 32 + (lane & 31), p.m - 1) * p.k;
+    col[i] = min(n0 + wn * (BM / 2) + i * 32 + (lane & 31), p.n - 1);
+    zc[i] = p.zero != nullptr && p.mode != kScalePerRow
+                ? static_cast<float>(p.zero[p.mode == kScalePerCol ? col[i] : p.const_index]) : 0.f;
+#pragma unroll
+    for (int j = 0; j < S; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  }
+#pragma unroll 1
+  for (int64_t kk = kb; kk < ke; kk += 2) {
+    const int64_t gk = min(kk + (lane >> 5), ke - 1);
+    const bool in = kk + (lane >> 5) < ke;
+    float rs = 1.f, rz = 0.f;
+    if (p.mode == kScalePerRow) {
+      rs = p.scale[gk];
+      if (p.zero != nullptr) rz = static_cast<float>(p.zero[gk]);
+    }
+    float av[S], bv[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      av[i] = in ? arow[i][gk] : 0.f;
+      const float w = static_cast<float>(p.q[gk * p.n + col[i]]) - zc[i] - rz;
+      bv[i] = in ? __fmul_rn(w, rs) : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int j = 0; j < S; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+  }
+}
+
+// Whether some raw sum of the wave calls for PlainSums: non-finite, or nonzero and so small (below
+// 2^-64) that parts below 2^-110 may have made it.
+template <int S>
+__device__ __forceinline__ bool NeedsPlainSums(const v16f (&acc)[S][S]) {
+  uint32_t largest = 0, smallest = 0xffffffffu;  // of the bits without the sign; a zero counts as largest
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int j = 0; j < S; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
+        largest = max(largest, u);
+        smallest = min(smallest, u - 1);
+      }
+  return __any(largest >= 0xff000000u || smallest < (uint32_t(127 - 64) << 24) - 1);
+}
+
+template <int BM, int kForm>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 2 : 3))) void GemmQ8Bf16Kernel(
     Q8GemmArgs p) {
   constexpr int kBufWords = Tile<BM>::kBufWords;
@@ -216,8 +356,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
   const int tn = in_band / rows_in_band;
   const int64_t m0 = static_cast<int64_t>(tm) * BM;
   const int64_t n0 = static_cast<int64_t>(tn) * BM;
-  const int64_t kb = static_cast<int64_t>(blockIdx.y) * p.k_per_split;
-  const int chunks = static_cast<int>((min(p.k, kb + p.k_per_split) - kb) / kBK);
+  const int64_t c0 = static_cast<int64_t>(blockIdx.y) * p.chunks_per_split;
+  const int64_t k_chunks = (p.k + kBK - 1) / kBK;
+  const int chunks = static_cast<int>(min(k_chunks, c0 + p.chunks_per_split) - c0);
+  const int pad = kForm == kPlain ? 0 : static_cast<int>(k_chunks * kBK - p.k);
 
   v16f acc[S][S], acc_ml[S][S];
 #pragma unroll
@@ -230,11 +372,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
         acc_ml[i][j][r] = 0.f;
       }
 
-  Panels<BM> regs[kStages];
+  ColConst cc;
+  LoadColConst<BM, kForm>(p, n0, tid, cc);
+  Panels<BM, kForm> regs[kStages];
 #pragma unroll
   for (int st = 0; st < kStages; ++st)
-    if (st < chunks) LoadPanels(p, m0, n0, kb + static_cast<int64_t>(st) * kBK, tid, regs[st]);
-  StorePanels(lds, tid, regs[0]);
+    if (st < chunks) LoadPanels(p, m0, n0, ChunkK<kForm>(c0 + st, pad), tid, regs[st]);
+  if (kForm != kPlain && c0 == 0 && pad != 0) {
+#pragma unroll
+    for (int i = 0; i < Tile<BM>::kARows; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (4 * (tid & 7) + t >= kBK - pad) regs[0].a[i][t] = 0.f;
+  }
+  StorePanels(lds, tid, regs[0], cc);
   __syncthreads();
   for (int base = 0; base < chunks; base += kStages) {
 #pragma unroll
@@ -245,9 +396,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
       // and LDS stores with this chunk's MFMAs. Past the end, the loads repeat the last chunk
       // and the store goes to the idle buffer; neither is used.
       const int nxt = min(ch + kStages, chunks - 1);
-      LoadPanels(p, m0, n0, kb + static_cast<int64_t>(nxt) * kBK, tid, regs[st]);
+      LoadPanels(p, m0, n0, ChunkK<kForm>(c0 + nxt, pad), tid, regs[st]);
       ComputeChunk<BM>(lds + (ch & 1) * kBufWords, lane, wm, wn, acc, acc_ml);
-      StorePanels(lds + ((ch + 1) & 1) * kBufWords, tid, regs[(st + 1) % kStages]);
+      StorePanels(lds + ((ch + 1) & 1) * kBufWords, tid, regs[(st + 1) % kStages], cc);
       if (BM == 128) {
         // Interleave: one MFMA, then a share of the conversion work and of the LDS stores.
 #pragma unroll
@@ -268,6 +419,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
 
+  if constexpr (kForm != kPlain) {
+    if (NeedsPlainSums<S>(acc))
+      PlainSums<BM>(p, m0, n0, ChunkK<kForm>(c0, pad), ChunkK<kForm>(c0 + chunks, pad), lane, wm, wn, acc);
+  }
   // Element r of a 32 x 32 tile sits at row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.
   if (p.partials != nullptr) {  // SplitReduceKernel adds the splits in order, scales, applies the epilogue
     float* part = p.partials + static_cast<int64_t>(blockIdx.y) * p.m * p.n;
@@ -289,7 +444,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
   for (int j = 0; j < S; ++j) {
     const int64_t col = n0 + wn * (BM / 2) + j * 32 + (lane & 31);
     if (col >= p.n) continue;
-    const float cs = p.scale[p.mode == kScalePerCol ? col : p.const_index];
+    const float cs = kForm == kRows ? 1.f : p.scale[p.mode == kScalePerCol ? col : p.const_index];
 #pragma unroll
     for (int i = 0; i < S; ++i)
 #pragma unroll
@@ -1091,13 +1246,55 @@ bool LaunchGemmQ8Small(const float* a, const Q8View& b, float* c, int64_t m, int
   return true;
 }
 
+namespace {
+
+// Tile side and K splits of GemmQ8Bf16Kernel: the cheapest by this estimate (us). A workgroup's
+// chunk takes kChunk128[w] (kChunk64[w]) with w workgroups on its CU, at most 2 (3) at once; a
+// split adds a launch and the partial sums' way through memory. Chunk times measured at
+// k = 4096, n = 4096: 128 tiles 1.0 us alone on a CU (m = 1000, no split: 129 us), 1.75 us two
+// together (m = 1000, two splits: 122 us); 64 tiles 0.6 / 0.8 / 1.06 us (m = 100, 333 and 333 in
+// two splits: 78.6, 101 and 73 us). m = 333: 128 tiles in 5 splits 52 us, in 2 / 3 / 4 / 8
+// splits 66 / 68 / 57 / 56, 64 tiles 101 / 73 / 72 / 74 us in 1 / 2 / 4 / 8 (what ran before: 64
+// tiles, no split).
+struct Q8Plan {
+  int bm;
+  int64_t splits;
+};
+
+Q8Plan PlanQ8Gemm(int64_t m, int64_t n, int64_t chunks, int64_t cus) {
+  constexpr double kChunk128[3] = {0, 1.0, 1.75};
+  constexpr double kChunk64[4] = {0, 0.6, 0.8, 1.06};
+  constexpr int64_t kMaxSplits = 16;
+  Q8Plan best{128, 1};
+  double best_us = 0;
+  for (const int bm : {128, 64}) {
+    const int64_t tiles = ((m + bm - 1) / bm) * ((n + bm - 1) / bm);
+    const int64_t cap = bm == 128 ? 2 : 3;
+    const double* us = bm == 128 ? kChunk128 : kChunk64;
+    for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(kMaxSplits, chunks / 3)); ++s) {
+      if (s > 1 && tiles * (s - 1) >= cap * cus) break;  // the CUs are full with fewer splits
+      const int64_t per_cu = (tiles * s + cus - 1) / cus;
+      double t = ((per_cu / cap) * us[cap] + us[per_cu % cap]) * static_cast<double>((chunks + s - 1) / s);
+      if (s > 1) t += 3.0 + static_cast<double>((2 * s + 1) * m * n) * 4e-6 / 4.0;
+      if (best_us == 0 || t < best_us) {
+        best_us = t;
+        best = Q8Plan{bm, s};
+      }
+    }
+  }
+  return best;
+}
+
+}  // namespace
+
 bool LaunchGemmQ8Bf16(const float* a, const Q8View& b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
                       hipStream_t stream, const RmsRequest* rms, bool* rms_done) {
   if (rms_done != nullptr) *rms_done = false;
-  if (b.q == nullptr || b.zero != nullptr || (b.mode != kScalePerCol && b.mode != kScaleConst)) return false;
-  if (m < 1 || k < kBK || n < 8 || k % kBK != 0 || n % 8 != 0) return false;
-  if (reinterpret_cast<uintptr_t>(a) % 16 != 0 || reinterpret_cast<uintptr_t>(b.q) % 8 != 0) return false;
-  if (b.bf16 != nullptr && GemmWantsBf16Image(m, k, n, b)) {
+  if (b.q == nullptr || m < 1 || k < kBK || n < 8) return false;
+  const bool plain = b.zero == nullptr && (b.mode == kScalePerCol || b.mode == kScaleConst) && k % kBK == 0 &&
+                     n % 8 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(b.q) % 8 == 0;
+  if (plain && b.bf16 != nullptr && GemmWantsBf16Image(m, k, n, b)) {
     const int64_t tiles_m = (m + kImgRows - 1) / kImgRows;
     const int64_t tiles_n = (n + kImgRows - 1) / kImgRows;
     const int64_t chunks = k / kBK;
@@ -1152,27 +1349,26 @@ bool LaunchGemmQ8Bf16(const float* a, const Q8View& b, float* c, int64_t m, int6
       return true;
     }
   }
-  if (LaunchGemmQ8Small(a, b, c, m, k, n, epi, stream, nullptr)) return true;
+  if (plain && LaunchGemmQ8Small(a, b, c, m, k, n, epi, stream, nullptr)) return true;
   Context& ctx0 = Ctx();
   const int64_t cus = ctx0.cu_count > 0 ? ctx0.cu_count : 256;
-  // 128 x 128 tiles when they give one per CU, else 64 x 64.
-  const int bm = ((m + 127) / 128) * ((n + 127) / 128) >= cus ? 128 : 64;
+  const int64_t chunks = (k + kBK - 1) / kBK;
+  const Q8Plan plan = PlanQ8Gemm(m, n, chunks, cus);
+  const int bm = plan.bm;
   const int64_t tiles_m = (m + bm - 1) / bm;
   const int64_t tiles_n = (n + bm - 1) / bm;
   const int64_t tiles = tiles_m * tiles_n;
   if (tiles * kBand > 0x7fffffff) return false;
-  // A grid short of one tile per CU splits K into ranges of whole chunks (at least 3 each),
-  // to about two workgroups per CU; a second kernel adds the partial sums in split order.
-  const int64_t chunks = k / kBK;
-  int64_t splits = 1;
-  if (tiles < cus) splits = std::max<int64_t>(1, std::min<int64_t>((2 * cus + tiles - 1) / tiles, chunks / 3));
-  const int64_t kper = (chunks + splits - 1) / splits * kBK;
-  splits = (k + kper - 1) / kper;
-  if (splits > 65535) return false;
+  // With a split K (ranges of whole chunks) a second kernel adds the partial sums in split order.
+  // Where the partial sums have no room (inside a capture, or the no-allocation scratch) K stays whole.
+  const int64_t cper = (chunks + plan.splits - 1) / plan.splits;
+  int64_t splits = (chunks + cper - 1) / cper;
+  if (splits > 1 && !ScratchReady(static_cast<size_t>(splits * m * n) * sizeof(float), kTempFlags, 0)) splits = 1;
   Q8GemmArgs args;
   args.a = a;
   args.q = b.q;
   args.scale = b.scale;
+  args.zero = b.zero;
   args.mode = b.mode;
   args.const_index = b.const_index;
   args.c = c;
@@ -1183,13 +1379,24 @@ bool LaunchGemmQ8Bf16(const float* a, const Q8View& b, float* c, int64_t m, int6
   args.tiles_n = static_cast<int32_t>(tiles_n);
   args.tiles = static_cast<int32_t>(tiles);
   args.tiles_per_xcd = static_cast<int32_t>((tiles + kXcds - 1) / kXcds);
-  args.k_per_split = kper;
+  args.chunks_per_split = splits > 1 ? cper : chunks;
   args.partials = nullptr;
   args.epi = epi;
   if (splits > 1) args.partials = static_cast<float*>(Workspace(static_cast<size_t>(splits * m * n) * sizeof(float)));
   const dim3 grid(static_cast<uint32_t>(args.tiles_per_xcd * kXcds), static_cast<uint32_t>(splits));
-  if (bm == 128) hipLaunchKernelGGL(GemmQ8Bf16Kernel<128>, grid, dim3(kThreads), 0, stream, args);
-  else hipLaunchKernelGGL(GemmQ8Bf16Kernel<64>, grid, dim3(kThreads), 0, stream, args);
+  const int form = plain ? kPlain : b.mode == kScalePerRow ? kRows : kCols;
+#define ACCEL_Q8_FORM(BM, F) \
+  if (form == F) hipLaunchKernelGGL((GemmQ8Bf16Kernel<BM, F>), grid, dim3(kThreads), 0, stream, args)
+  if (bm == 128) {
+    ACCEL_Q8_FORM(128, kPlain);
+    ACCEL_Q8_FORM(128, kCols);
+    ACCEL_Q8_FORM(128, kRows);
+  } else {
+    ACCEL_Q8_FORM(64, kPlain);
+    ACCEL_Q8_FORM(64, kCols);
+    ACCEL_Q8_FORM(64, kRows);
+  }
+#undef ACCEL_Q8_FORM
   Check(hipGetLastError(), "GemmQ8Bf16Kernel launch");
   if (splits > 1) LaunchSplitReduce(args.partials, static_cast<int32_t>(splits), m, n, c, b.mode, b.scale, b.const_index,
                                     epi, stream);

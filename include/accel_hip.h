@@ -130,10 +130,10 @@ ACCEL_HIP_API int accel_hip_matmul(AccelHipBuffer a, AccelHipBuffer b, AccelHipB
  * Device pointers; a NULL plane reads the float pointer. Either side may be quantized.
  * w = (float(q) - float(zero)) * scale at the plane's coordinate. m <= 16: the int8 GEMV
  * (VALU for m <= 2, exact bf16-split products on the matrix cores for 3 <= m <= 16). Above
- * that, an int8 weight with per-column or whole-tensor scale, no zero points and k % 32 == 0
- * runs on the bf16 matrix cores with the activation split exactly into three bf16 parts (the
- * weight staged once as bf16); other planes on the fp32 MFMA GEMM with the int8 panel
- * dequantized in LDS. */
+ * that, an int8 weight with k >= 32 and n >= 8 runs on the bf16 matrix cores with the activation
+ * split exactly into three bf16 parts (with a per-column or whole-tensor scale, no zero points,
+ * k % 32 == 0 and n % 8 == 0 the weight is staged once as bf16); smaller ones on the fp32 MFMA
+ * GEMM with the int8 panel dequantized in LDS. */
 ACCEL_HIP_API int accel_hip_matmul_quantized(const float* a, const AccelHipQuantPlane* a_quant, const float* b,
                                              const AccelHipQuantPlane* b_quant, float* c, int64_t m, int64_t k,
                                              int64_t n);
