@@ -353,6 +353,10 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
 // nothing, for sizes it does not take (n < 4, or sides of 2^28 and more).
 bool LaunchGemvF32(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
                    hipStream_t stream);
+// C[m, n] = A[m, k] @ B[k, n] in fp32 from six bf16 part products (gemm_f32_parts.hip). False,
+// launching nothing, for sizes it does not take (k < 32).
+bool LaunchGemmF32Parts(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
+                        hipStream_t stream);
 // The int8-weight GEMM on the bf16 matrix cores (exact products, activations split into
 // three bf16 parts): k >= 32, n >= 8 (a grid that leaves CUs idle splits K where the workspace
 // for it can be had). The staged-copy kernels take k % 32 == 0, n % 8 == 0, A 16-byte and q 8-byte

@@ -1,6 +1,8 @@
 // fp32 GEMM on the matrix cores: C[m, n] = A[m, k] @ B[k, n] (+ fused epilogue), B either
 // fp32 (Device::MatMul, src/sim_device.cc:185-196) or an int8 plane dequantized panel by
-// panel into LDS (accel::MatMulQuantized for m > 16 with k < 32 or n < 8, src/sim_device.cc:541-602).
+// panel into LDS (accel::MatMulQuantized, src/sim_device.cc:541-602). GemmKernel takes what the
+// bf16-part kernels do not: k < 32, or int8 with n < 8 (m > 16); GemmF32SplitBf16Kernel further
+// down small grids of whole tiles; gemm_f32_parts.hip every other fp32 product.
 //
 // Bound: MFMA (fp32, v_mfma_f32_32x32x2_f32). 2*m*n*k flops per call.
 //
@@ -745,7 +747,14 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
     int64_t wsplits = wtiles < cus ? std::max<int64_t>(1, std::min<int64_t>((cus + wtiles - 1) / wtiles, k / (4 * unit)))
                                    : 1;
     while (wsplits > 1 && k % (wsplits * unit) != 0) --wsplits;
-    if (k % (wsplits * unit) == 0 && wtiles <= 0x7fffffff && m <= 0x7fffffff && n <= 0x7fffffff && k <= 0x7fffffff) {
+    // A grid that leaves half the CUs idle is faster in more splits on GemmF32PartsKernel (m x k x n:
+    // 64 x 1536 x 576 20.4 us here, 11.3 there; 256 x 512 x 2048, half of the CUs, 11.0 and 13.0; the
+    // MLP's 256 x 1024 x 4096 16.9 and 26.6). A round of 128 tiles is faster there too (1024 x 4096 x
+    // 4096 206 us, 173 there), but its K chains are twice as long: error 1.9e-7 here, 2.7e-7 there. K
+    // ranges of exactly 1024 (the unrolled form) stay here at any grid (128 x 1024 x 1024 14.3 us,
+    // 11.1 there): a caller may count on their weight's staged parts.
+    const bool keep = 2 * wtiles * wsplits >= cus || k == wsplits * 4 * unit;
+    if (k % (wsplits * unit) == 0 && keep && wtiles <= 0x7fffffff && m <= 0x7fffffff && n <= 0x7fffffff && k <= 0x7fffffff) {
       WsArgs ws;
       ws.a = a;
       ws.b = b;
@@ -780,6 +789,7 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
       return false;
     }
   }
+  if (!q8 && LaunchGemmF32Parts(a, b, c, m, k, n, epi, stream)) return false;
   if (tiles_for(128, 128) < 2 * cus) {
     bm = 64;
     bn = 64;

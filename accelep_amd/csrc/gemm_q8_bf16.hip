@@ -35,7 +35,7 @@
 //    panel gain a subtraction, a ragged k zeroes part of its first chunk, loads need no alignment.
 //    They had run on the fp32 matrix cores with each panel dequantized on the way into LDS:
 //    333 x 4096 x 4096 with zero points 223 us (50 TFLOP/s) -> 55, with a per-row scale 227 -> 56,
-//    333 x 4095 x 4097 440 -> 62, 2000 x 2047 x 14335 1651 -> 405, 2000 x 2048 x 14336 with zero
+//    333 x 4095 x 4097 440 -> 77, 2000 x 2047 x 14335 1651 -> 407, 2000 x 2048 x 14336 with zero
 //    points 1011 -> 383. Error against float64 at k = 4096: 1.1e-6 -> 1.1e-7 .. 2.5e-7.
 #include "device_common.h"
 
