@@ -223,12 +223,12 @@ bool GemmWantsSmall(int64_t m, int64_t k, int64_t n, const Q8View& v);
 // without the grid condition on m).
 bool GemmBf16Stageable(int64_t k, int64_t n, const Q8View& v);
 // Whether LaunchGemvQ8 takes an m-row product with this k, n and weight view from the
-// group-interleaved copy (the caller stages that copy instead of the 8-column tiles): 3 <= m
-// <= 16, whole 32-row blocks, no zero points or per-row scale, and for m <= 4 a product large
-// enough to give every CU a workgroup of the split-bf16 kernel (a smaller one runs on the
-// narrow kernel's tiles, one workgroup per tile and no K-split exchange).
+// group-interleaved copy (the caller stages that copy): 3 <= m <= 16, whole 32-row blocks, no zero
+// points or per-row scale, a large matrix; or from the 8-column tiles (m <= 4, the larger m only
+// while the matrix is small). Otherwise W is read in place.
 constexpr int64_t kGemvGroupMinM = 3;
 bool GemvWantsGroups(int64_t m, int64_t k, int64_t n, const Q8View& v);
+bool GemvWantsTiles(int64_t m, int64_t k, int64_t n, const Q8View& v);
 
 struct Epilogue {
   float alpha = 1.f;
@@ -307,11 +307,14 @@ constexpr int64_t kGemvAttnMaxPairs = 2048;  // heads x splits of GemvPrologue::
 
 // C[m, n] = A[m, k] @ dequant(Bq)[k, n] for m <= 16 (int8 GEMV). With b.grouped (and no zero
 // points or per-row scale, k % 32 == 0, A 16-byte aligned) the split-bf16 MFMA kernel runs;
-// with b.tiled the 8-column tile kernels; otherwise W is read in place. A prologue needs m == 1,
+// with b.tiled the 8-column tile kernels (GemvWantsTiles); otherwise W is read in place. A prologue needs m == 1,
 // staged tiles, a per-column or whole-tensor scale without zero points and k <=
 // kGemvPrologueMaxK.
 void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
                   hipStream_t stream, const GemvPrologue* prologue = nullptr);
+// The same product of any plane with W read in place (no staged copy, no prologue).
+void LaunchGemvQ8InPlace(const float* a, const Q8View& b, float* c, int64_t m, int64_t k, int64_t n,
+                         const Epilogue& epi, hipStream_t stream);
 // Whether an m = 1 GEMV of this shape (on staged tiles, aligned pairs, per-column or tensor scale,
 // identity epilogue) runs one wave per tile: an even k <= 1024 over at least 8 tiles per CU. There
 // the norm-after prologue may come with the greedy keys and the advance.

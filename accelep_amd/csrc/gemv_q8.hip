@@ -22,12 +22,9 @@
 // group-interleaved staged copy of the tiles, exact products on v_mfma_f32_16x16x32_bf16
 // with each activation split into three bf16 parts, split-K summed in split order by the
 // last workgroup of each column group to arrive (no second kernel).
-// Wide kernel (the other 4 < m <= 16 cases): W in place, 256-column tiles, 16 lanes per
-// 256-byte row segment, 4 rows per wave load feed v_mfma_f32_16x16x4_f32 as its K = 4; A
-// staged in LDS.
-// Split-K of the narrow and wide kernels (only where the tile count cannot fill the GPU):
-// each split writes its partial sums to the workspace and a second kernel adds them in
-// split order.
+// The other cases: gemv_q8_inplace.hip.
+// Split-K of the narrow kernel (only where the tile count cannot fill the GPU): each split
+// writes its partial sums to the workspace and a second kernel adds them in split order.
 #include "device_common.h"
 
 namespace accel_hip {
@@ -65,48 +62,10 @@ struct GemvArgs {
   GemvPrologue pro;  // narrow m = 1 kernel with kAOp != 0
 };
 
-// The 16 bytes at columns [col, col + 16) of one row (`row` must point inside W); zero past
-// n or when !valid. The 16-byte form loads unconditionally from a clamped column (n >= 16
-// there) and selects, so no branch forces an early wait on the load.
-template <bool kVec>
-__device__ __forceinline__ uint4 LoadRow16(const int8_t* row, int64_t col, int64_t n, bool valid) {
-  if (kVec) {
-    // Columns past n read a clamped in-range chunk: their sums land in columns >= n, which
-    // are never stored. Invalid rows are neutralized by a zero A operand at use.
-    const int64_t cc = col < n ? col : n - 16;
-    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + cc));
-    return make_uint4(v[0], v[1], v[2], v[3]);
-  }
-  uint32_t w[4] = {0, 0, 0, 0};
-  if (valid) {
-    for (int b = 0; b < 16; ++b) {
-      if (col + b < n) w[b >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(row[col + b])) << (8 * (b & 3));
-    }
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
-__device__ __forceinline__ uint32_t Word(const uint4& v, int d) {
-  return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w;
-}
-
 __device__ __forceinline__ float ColScale(const GemvArgs& p, int64_t col) {
   if (p.mode == kScalePerCol) return p.scale[col];
   if (p.mode == kScaleConst) return p.scale[p.const_index];
   return 1.f;  // per-row scale was folded into A
-}
-
-// Zero points of the 16 columns [col, col + 16) (per-column or whole-tensor), as floats.
-template <bool kZero>
-__device__ __forceinline__ void ColumnZeros(const GemvArgs& p, int64_t col, float (&zc)[16]) {
-  for (int j = 0; j < 16; ++j) zc[j] = 0.f;
-  if (!kZero) return;
-  if (p.mode == kScalePerCol) {
-    for (int j = 0; j < 16; ++j) zc[j] = (col + j < p.n) ? static_cast<float>(p.zero[col + j]) : 0.f;
-  } else if (p.mode == kScaleConst) {
-    const float z = static_cast<float>(p.zero[p.const_index]);
-    for (int j = 0; j < 16; ++j) zc[j] = z;
-  }
 }
 
 // Stores one finished sum: to the split's partials, or scaled + epilogue into C.
@@ -804,141 +763,6 @@ __global__ __launch_bounds__(64 * kWaveTileWaves) void GemvWaveTileKernel(const 
   }
 }
 
-// ---- wide kernel: 4 < m <= 16 ----------------------------------------------------------------
-constexpr int kWideThreads = 256;
-constexpr int kWideWaves = kWideThreads / 64;
-constexpr int kWideTile = 256;
-constexpr int kWideMaxRows = 1024;
-constexpr int kWideUnroll = 4;
-
-// One step of the wide kernel: row group g = g0 + u * waves holds rows 4g .. 4g + 3, lane row
-// l / 16 of it; rows past `rows` read a clamped row and are zeroed through A.
-template <bool kVec>
-__device__ __forceinline__ void WideLoad(const GemvArgs& p, const int8_t* wbase, int64_t col, int rows, int groups,
-                                         int g0, int lane_row, uint4 (&w)[kWideUnroll]) {
-#pragma unroll
-  for (int u = 0; u < kWideUnroll; ++u) {
-    const int g = g0 + u * kWideWaves;
-    const int r = g * 4 + lane_row;
-    const bool valid = g < groups && r < rows;
-    const int rc = valid ? r : rows - 1;
-    w[u] = LoadRow16<kVec>(wbase + static_cast<int64_t>(rc) * p.n, col, p.n, valid);
-  }
-}
-
-template <bool kZero, bool kRowScale>
-__device__ __forceinline__ void WideStep(const GemvArgs& p, const float* smem, int64_t k0, int rows, int groups, int g0,
-                                         int lane_row, int lane_col, const float (&zc)[16],
-                                         const uint4 (&w)[kWideUnroll], v4f (&acc)[16]) {
-#pragma unroll
-  for (int u = 0; u < kWideUnroll; ++u) {
-    const int g = g0 + u * kWideWaves;
-    const int r = g * 4 + lane_row;
-    const bool valid = g < groups && r < rows;
-    const int rc = valid ? r : rows - 1;
-    const float a = smem[rc * 16 + lane_col];  // A[l % 16][row of l]
-    const float av = valid ? a : 0.f;
-    const float zr = (kZero && kRowScale) ? static_cast<float>(p.zero[k0 + rc]) : 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      float b = ByteToFloat(Word(w[u], t >> 2), t & 3);
-      if (kZero) b = b - (zc[t] + zr);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, b, acc[t], 0, 0, 0);
-    }
-  }
-}
-
-template <bool kVec, bool kZero, bool kRowScale>
-__global__ __launch_bounds__(kWideThreads) void GemvWideKernel(GemvArgs p) {
-  __shared__ __align__(16) float smem[16 * kWideMaxRows];  // A stage [row][16]; reused for the wave sums
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int tile = blockIdx.x;
-  if (tile >= p.tiles) return;
-  const int split = blockIdx.y;
-  const int64_t k0 = static_cast<int64_t>(split) * p.rows_per_split;
-  const int rows = static_cast<int>(min(p.rows_per_split, p.k - k0));
-
-  // A stage: smem[r * 16 + mm] = A[mm][k0 + r] (times the row's scale when per-row), 0 for
-  // mm >= m. Thread r reads its row's 16 values down A's columns (consecutive threads,
-  // consecutive addresses) and issues all of them before storing any, so the stage costs one
-  // memory round trip per 256 rows instead of one per element.
-  for (int r0 = 0; r0 < rows; r0 += kWideThreads) {
-    const int r = r0 + tid;
-    const int rc = r < rows ? r : rows - 1;
-    float v[16];
-#pragma unroll
-    for (int mm = 0; mm < 16; ++mm) {
-      const int64_t mc = mm < p.m ? mm : p.m - 1;  // a valid row; zeroed below
-      v[mm] = p.a[mc * p.k + k0 + rc];
-    }
-    const float rs = kRowScale ? p.scale[k0 + rc] : 1.f;
-    if (r < rows) {
-#pragma unroll
-      for (int mm = 0; mm < 16; mm += 4) {
-        float4 q;
-        q.x = mm + 0 < p.m ? (kRowScale ? __fmul_rn(v[mm + 0], rs) : v[mm + 0]) : 0.f;
-        q.y = mm + 1 < p.m ? (kRowScale ? __fmul_rn(v[mm + 1], rs) : v[mm + 1]) : 0.f;
-        q.z = mm + 2 < p.m ? (kRowScale ? __fmul_rn(v[mm + 2], rs) : v[mm + 2]) : 0.f;
-        q.w = mm + 3 < p.m ? (kRowScale ? __fmul_rn(v[mm + 3], rs) : v[mm + 3]) : 0.f;
-        *reinterpret_cast<float4*>(&smem[r * 16 + mm]) = q;
-      }
-    }
-  }
-  __syncthreads();
-
-  const int lane_row = lane >> 4;  // MFMA k of this lane
-  const int lane_col = lane & 15;  // MFMA column of this lane
-  const int64_t col = static_cast<int64_t>(tile) * kWideTile + lane_col * 16;
-  float zc[16];
-  ColumnZeros<kZero>(p, col, zc);
-  v4f acc[16];
-#pragma unroll
-  for (int t = 0; t < 16; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  const int groups = (rows + 3) >> 2;
-  const int8_t* wbase = p.q + k0 * p.n;
-  // The next step's rows are requested before this step's MFMAs (one set in flight while
-  // one is multiplied).
-  constexpr int kStride = kWideWaves * kWideUnroll;
-  uint4 wn[kWideUnroll];
-  WideLoad<kVec>(p, wbase, col, rows, groups, wave, lane_row, wn);
-  for (int g0 = wave; g0 < groups; g0 += kStride) {
-    uint4 w[kWideUnroll];
-#pragma unroll
-    for (int u = 0; u < kWideUnroll; ++u) w[u] = wn[u];
-    if (g0 + kStride < groups) WideLoad<kVec>(p, wbase, col, rows, groups, g0 + kStride, lane_row, wn);
-    WideStep<kZero, kRowScale>(p, smem, k0, rows, groups, g0, lane_row, lane_col, zc, w, acc);
-  }
-  __syncthreads();  // A stage done; smem becomes [wave][16][kWideTile]
-  // Lane l holds m = 4*(l/16) + r, column 16*(l%16) + t.
-  for (int r = 0; r < 4; ++r)
-    for (int t = 0; t < 16; ++t) smem[(wave * 16 + 4 * lane_row + r) * kWideTile + lane_col * 16 + t] = acc[t][r];
-  __syncthreads();
-  const int64_t out_col = static_cast<int64_t>(tile) * kWideTile + tid;
-  if (out_col >= p.n) return;
-  // All 16 rows' wave sums are read at once (one LDS round trip), then stored.
-  float sums[16];
-#pragma unroll
-  for (int mm = 0; mm < 16; ++mm) {
-    float s = smem[mm * kWideTile + tid];
-#pragma unroll
-    for (int wv = 1; wv < kWideWaves; ++wv) s = s + smem[(wv * 16 + mm) * kWideTile + tid];
-    sums[mm] = s;
-  }
-  if (p.splits > 1) {
-    float* dst = p.partials + static_cast<int64_t>(split) * p.m * p.n + out_col;
-#pragma unroll
-    for (int mm = 0; mm < 16; ++mm)
-      if (mm < p.m) dst[mm * p.n] = sums[mm];
-    return;  // SplitReduceKernel applies the scale and the epilogue
-  }
-#pragma unroll
-  for (int mm = 0; mm < 16; ++mm)
-    if (mm < p.m) Emit(p, split, mm, out_col, sums[mm]);
-}
-
 // ---- split-bf16 MFMA kernel: 1 < m <= 16, group-interleaved tiles, k a multiple of 32 ---------
 // The products run on v_mfma_f32_16x16x32_bf16 (A: 16 rows x 32 k, B: 32 k x 16 columns)
 // without rounding either operand:
@@ -1325,14 +1149,27 @@ int64_t CuCount() {
 
 }  // namespace
 
+// Least elements for the staged copies of 3 to 16 rows. Below it W is read in place by shorter
+// splits of K (m = 8, 16: 4096 x 8192 12.6, 13.6 us on the groups, 11.9, 13.1 in place; 4096 x
+// 4096 11.9, 12.8 and 8.8, 9.4; 576 x 3072 7.3, 7.7 and 4.6, 4.8), above it the groups stream
+// better (2048 x 14336 10.6, 11.3 and 11.2, 12.0; 4096 x 14336 15.6, 16.6 and 16.9, 17.7).
+constexpr int64_t kGroupMinElems = int64_t(28) << 20;
+
+bool GroupForm(int64_t k, const Q8View& v) {
+  return k % kGemvGroupRows == 0 && v.zero == nullptr && (v.mode == kScalePerCol || v.mode == kScaleConst);
+}
+
 bool GemvWantsGroups(int64_t m, int64_t k, int64_t n, const Q8View& v) {
-  if (m < kGemvGroupMinM || m > 16 || k % kGemvGroupRows != 0 || v.zero != nullptr ||
-      (v.mode != kScalePerCol && v.mode != kScaleConst))
-    return false;
-  if (m > 4) return true;  // the narrow kernel takes m <= 4 only
-  int64_t groups = 0, splits = 0;
-  SplitBf16Grid(k, n, CuCount(), &groups, &splits);
-  return groups * splits >= CuCount();
+  return m >= kGemvGroupMinM && m <= 16 && k * n >= kGroupMinElems && GroupForm(k, v);
+}
+
+// The narrow kernel's VALU work grows with m: three or four rows take it only while W is small
+// (m = 4: 4096 x 4096 6.9 us against 8.4 in place and 10.8 on the groups, 4096 x 6144 with zero
+// points 9.2 against 10.7; 2048 x 14336 with zero points 14.4 against 12.0). A plane of the
+// groups' form goes in place from 20 Mi elements (4096 x 6144 9.8 us in place, 3072 x 8192 8.9).
+bool GemvWantsTiles(int64_t m, int64_t k, int64_t n, const Q8View& v) {
+  if (m <= 2) return true;
+  return m <= 4 && k * n < (GroupForm(k, v) ? int64_t(20) << 20 : kGroupMinElems);
 }
 
 bool GemvWaveTileApplies(int64_t m, int64_t k, int64_t n) {
@@ -1363,18 +1200,22 @@ void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t 
   Context& ctx0 = Ctx();
   const int64_t cus = ctx0.cu_count > 0 ? ctx0.cu_count : 256;
   // The narrow kernel reads the staged column tiles (and indexes rows in 32 bits); without
-  // them the wide kernel, which reads W in place, takes any m <= 16.
+  // them the in-place kernel takes any m <= 16.
   const bool zero = b.zero != nullptr;
   const bool row_scale = b.mode == kScalePerRow;
   // The split-bf16 MFMA kernel: group-interleaved copy, whole 32-row blocks, A 16-byte aligned.
   const bool split_bf16 = m > 1 && b.grouped != nullptr && !zero && !row_scale && a_op == kAOpNone &&
                           k % kSplitBlockRows == 0 && k < (int64_t(1) << 28) && m * n <= 0x7fffffff &&
                           reinterpret_cast<uintptr_t>(a) % 16 == 0 && (b.mode == kScalePerCol || b.mode == kScaleConst);
-  const bool narrow = !split_bf16 && m <= 4 && b.tiled != nullptr && k < (int64_t(1) << 28);
+  const bool narrow = !split_bf16 && b.tiled != nullptr && k < (int64_t(1) << 28) && GemvWantsTiles(m, k, n, b);
   if (side && !narrow)
     Fail(ACCEL_HIP_INVALID_ARGUMENT, "GEMV greedy keys and advance need the m = 1 kernel (m = 1, staged tiles)");
-  const int64_t tile_cols = narrow || split_bf16 ? kNarrowTile : kWideTile;
-  const int64_t tiles = (n + tile_cols - 1) / tile_cols;
+  if (!narrow && !split_bf16) {
+    if (a_op != kAOpNone) Fail(ACCEL_HIP_INVALID_ARGUMENT, "GEMV input prologue needs the staged tiles");
+    LaunchGemvQ8InPlace(a, b, c, m, k, n, epi, stream);
+    return;
+  }
+  const int64_t tiles = (n + kNarrowTile - 1) / kNarrowTile;
   int64_t splits = 1;
   int64_t rows = k;
   if (split_bf16) {
@@ -1382,7 +1223,7 @@ void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t 
     SplitBf16Grid(k, n, cus, &groups, &splits);
     const int64_t blocks = k / kSplitBlockRows;
     rows = (blocks + splits - 1) / splits * kSplitBlockRows;
-  } else if (narrow) {
+  } else {
     // One workgroup per tile over all of K, unless the tiles leave the CUs short of work on a
     // K of several batches: then K is split so that about four workgroups run per CU.
     const int64_t step_rows = m == 1 ? NarrowShape<1>::kStepRows : NarrowShape<2>::kStepRows;
@@ -1391,13 +1232,6 @@ void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t 
       splits = std::min<int64_t>((4 * cus + tiles - 1) / tiles, k / batch_rows);
     rows = (k + splits - 1) / splits;
     rows = (rows + step_rows - 1) / step_rows * step_rows;
-  } else {
-    // About 1.75 workgroups per CU (measured best for 4096 x 14336 at m = 16), and no split
-    // longer than the A stage.
-    splits = std::max<int64_t>((7 * cus / 4 + tiles - 1) / tiles, (k + kWideMaxRows - 1) / kWideMaxRows);
-    splits = std::min<int64_t>(splits, std::max<int64_t>(1, (k + 255) / 256));
-    rows = (k + splits - 1) / splits;
-    rows = std::min<int64_t>((rows + 15) / 16 * 16, kWideMaxRows);
   }
   splits = (k + rows - 1) / rows;
   if (a_op != kAOpNone && splits != 1) Fail(ACCEL_HIP_INVALID_ARGUMENT, "GEMV input prologue needs one split");
@@ -1446,7 +1280,7 @@ void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t 
     else
       hipLaunchKernelGGL(GemvSplitBf16Kernel<false>, sgrid, dim3(kSplitThreads), 0, stream, b.grouped, a, args.partials,
                          args.arrivals, m32, k32, rows32, splits32, pairs32, args);
-  } else if (narrow) {
+  } else {
     const bool pair_a = (k % 2 == 0) && (reinterpret_cast<uintptr_t>(a) % 8 == 0);
     // The staged prologue row lives in LDS (16-byte aligned), so only an even k is needed
     // there; the norm-after form reads x and the norm weight in pairs from memory.
@@ -1599,19 +1433,6 @@ void LaunchGemvQ8(const float* a, const Q8View& b, float* c, int64_t m, int64_t 
       LaunchNarrow<2>(args, grid, zero, row_scale, pair_a, stream);
     } else {
       LaunchNarrow<4>(args, grid, zero, row_scale, pair_a, stream);
-    }
-  } else {
-    const bool vec = (n % 16 == 0) && (reinterpret_cast<uintptr_t>(b.q) % 16 == 0);
-    const dim3 block(kWideThreads);
-    switch ((vec ? 4 : 0) | (zero ? 2 : 0) | (row_scale ? 1 : 0)) {
-#define ACCEL_GEMV_CASE(V, Z, R) \
-  case (V ? 4 : 0) | (Z ? 2 : 0) | (R ? 1 : 0): \
-    hipLaunchKernelGGL((GemvWideKernel<V, Z, R>), grid, block, 0, stream, args); \
-    break;
-      ACCEL_GEMV_CASE(true, true, true) ACCEL_GEMV_CASE(true, true, false) ACCEL_GEMV_CASE(true, false, true)
-      ACCEL_GEMV_CASE(true, false, false) ACCEL_GEMV_CASE(false, true, true) ACCEL_GEMV_CASE(false, true, false)
-      ACCEL_GEMV_CASE(false, false, true) ACCEL_GEMV_CASE(false, false, false)
-#undef ACCEL_GEMV_CASE
     }
   }
   Check(hipGetLastError(), "GEMV launch");

@@ -223,7 +223,7 @@ struct Model {
         LaunchExactMatmul(a, nullptr, v, c, m, w.in, w.out, e, ctx.stream);
       } else if (m <= 16) {
         if (GemvWantsGroups(m, w.in, w.out, v)) v.grouped = StagedGroupTiles(v.q, w.in, w.out, ctx.stream);
-        else if (m <= 4) v.tiled = StagedColumnTiles(v.q, w.in, w.out, ctx.stream);
+        else if (GemvWantsTiles(m, w.in, w.out, v)) v.tiled = StagedColumnTiles(v.q, w.in, w.out, ctx.stream);
         LaunchGemvQ8(a, v, c, m, w.in, w.out, e, ctx.stream);
       } else {
         if (GemmWantsSmall(m, w.in, w.out, v)) v.bf16x16 = StagedBf16x16(v.q, w.in, w.out, ctx.stream);

@@ -129,7 +129,8 @@ ACCEL_HIP_API int accel_hip_matmul(AccelHipBuffer a, AccelHipBuffer b, AccelHipB
 /* accel::MatMulQuantized (include/accel/runtime.h:124-125; src/sim_device.cc:541-602).
  * Device pointers; a NULL plane reads the float pointer. Either side may be quantized.
  * w = (float(q) - float(zero)) * scale at the plane's coordinate. m <= 16: the int8 GEMV
- * (VALU for m <= 2, exact bf16-split products on the matrix cores for 3 <= m <= 16). Above
+ * (VALU for m <= 2 and small matrices at m <= 4, else exact bf16-split products on the matrix
+ * cores, from the group-interleaved copy where a large matrix has one, else in place). Above
  * that, an int8 weight with k >= 32 and n >= 8 runs on the bf16 matrix cores with the activation
  * split exactly into three bf16 parts (with a per-column or whole-tensor scale, no zero points,
  * k % 32 == 0 and n % 8 == 0 the weight is staged once as bf16); smaller ones on the fp32 MFMA
@@ -146,8 +147,8 @@ ACCEL_HIP_API int accel_hip_matmul_quantized(const float* a, const AccelHipQuant
  * weight's allocation is freed or written. Refused (ACCEL_HIP_RUNTIME_ERROR) during a graph
  * capture; ACCEL_HIP_INVALID_ARGUMENT for a layout the plane cannot take or a weight outside
  * this library's heap. *staged (if not NULL) receives the layouts built. */
-#define ACCEL_HIP_STAGE_GEMV_TILES 1u  /* 8-column tiles: the int8 GEMV at m <= 4 where groups are not taken */
-#define ACCEL_HIP_STAGE_GEMV_GROUPS 2u /* group-interleaved tiles: the bf16-split GEMV, 3 <= m <= 16 */
+#define ACCEL_HIP_STAGE_GEMV_TILES 1u  /* 8-column tiles: the int8 GEMV at m <= 2, and at m <= 4 for small matrices */
+#define ACCEL_HIP_STAGE_GEMV_GROUPS 2u /* group-interleaved tiles: the bf16-split GEMV, 3 <= m <= 16, from 28 Mi weights */
 #define ACCEL_HIP_STAGE_GEMM_BF16 4u   /* bf16 in MFMA operand order: the int8-weight GEMM, m > 16 */
 #define ACCEL_HIP_STAGE_GEMM_SMALL 8u  /* bf16 in the small GEMM's operand order: m > 16, k <= 768 */
 #define ACCEL_HIP_STAGE_ALL 15u
