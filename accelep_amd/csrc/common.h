@@ -353,9 +353,17 @@ struct RmsRequest {
 bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, int64_t m, int64_t k, int64_t n,
                    const Epilogue& epi, hipStream_t stream, const RmsRequest* rms = nullptr, bool stage_b = false);
 // C[m, n] = A[m, k] @ B[k, n] for m <= 16, B fp32 read in place (gemv_f32.hip). False, launching
-// nothing, for sizes it does not take (n < 4, or sides of 2^28 and more).
+// nothing, for sizes it does not take (n < 4, or sides of 2^28 and more). A prologue (m = 1, k <=
+// kGemvPrologueMaxK) is one of GemvPrologue's input transforms: rms_weight with the norm applied
+// after the product (rms_after there), and with it the SiLU of columns [0, epi.split[0]), or mul_up.
+struct F32Prologue {
+  const float* rms_weight = nullptr;
+  float rms_eps = 0.f;
+  bool silu_split0 = false;
+  const float* mul_up = nullptr;
+};
 bool LaunchGemvF32(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,
-                   hipStream_t stream);
+                   hipStream_t stream, const F32Prologue* prologue = nullptr);
 // C[m, n] = A[m, k] @ B[k, n] in fp32 from six bf16 part products (gemm_f32_parts.hip). False,
 // launching nothing, for sizes it does not take (k < 32).
 bool LaunchGemmF32Parts(const float* a, const float* b, float* c, int64_t m, int64_t k, int64_t n, const Epilogue& epi,

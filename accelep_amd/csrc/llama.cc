@@ -241,6 +241,15 @@ struct Model {
   bool Fusable(const Linear& w, int64_t m) const {
     return (fuse & 1) != 0 && m == 1 && !w.q.empty() && !Ctx().exact_products && w.in <= kGemvPrologueMaxK;
   }
+  // The same for an fp32 weight.
+  bool FusableF32(const Linear& w, int64_t m) const {
+    return (fuse & 1) != 0 && m == 1 && !w.f.empty() && !Ctx().exact_products && w.in <= kGemvPrologueMaxK &&
+           w.out >= 4 && w.out < (int64_t(1) << 28);
+  }
+  void ApplyPrologueF32(const Linear& w, const float* x, float* c, const Epilogue& e, const F32Prologue& pro) {
+    if (!LaunchGemvF32(x, w.f.as<float>(), c, 1, w.in, w.out, e, Ctx().stream, &pro))
+      Fail(ACCEL_HIP_RUNTIME_ERROR, "fp32 GEMV prologue planned for a product that cannot take it");
+  }
   // The o-projection may read the split attention's partials (fuse bit 2).
   bool SplitAttention(const Linear& o) const {
     return (fuse & 4) != 0 && !o.q.empty() && !Ctx().exact_products && o.in <= kGemvPrologueMaxK &&
@@ -271,6 +280,14 @@ struct Model {
       pro.rms_after = true;
       pro.silu_split0 = silu_split0;
       ApplyPrologue(w, x, c, e, pro);
+      return;
+    }
+    if (FusableF32(w, m)) {
+      F32Prologue pro;
+      pro.rms_weight = norm.as<float>();
+      pro.rms_eps = cfg.eps;
+      pro.silu_split0 = silu_split0;
+      ApplyPrologueF32(w, x, c, e, pro);
       return;
     }
     Q8View sv;
@@ -310,6 +327,12 @@ struct Model {
       ApplyPrologue(w, g, c, e, pro);
       return;
     }
+    if (silu_done && FusableF32(w, m)) {
+      F32Prologue pro;
+      pro.mul_up = u;
+      ApplyPrologueF32(w, g, c, e, pro);
+      return;
+    }
     if (silu_done) {
       Q8View sv;
       SmallPrologue pro;
@@ -332,6 +355,7 @@ struct Model {
       return SmallFusable(l.gu, m, gv) && SmallFusable(l.down, m, dv) && aligned(hidden.as<float>()) &&
              aligned(l.post_norm.as<float>()) && aligned(gate.as<float>()) && aligned(up.as<float>());
     }
+    if (FusableF32(l.gu, m)) return FusableF32(l.down, m);
     return Fusable(l.gu, m) && l.gu.out <= kFusedNormMaxOut && l.gu.in % 2 == 0 && Fusable(l.down, m) &&
            l.down.in % 2 == 0;
   }
@@ -357,6 +381,13 @@ struct Model {
       pro.advance = state;
       ApplyPrologue(lm_head, x, logits.as<float>(), Epilogue{}, pro);
       return state != nullptr;
+    }
+    if (FusableF32(lm_head, 1)) {
+      F32Prologue pro;
+      pro.rms_weight = final_norm.as<float>();
+      pro.rms_eps = cfg.eps;
+      ApplyPrologueF32(lm_head, x, logits.as<float>(), Epilogue{}, pro);
+      return false;
     }
     LaunchRmsNormRows(x, final_norm.as<float>(), normed.as<float>(), 1, cfg.hidden, cfg.eps, stream());
     Mark(kMarkHeadNorm);

@@ -112,7 +112,7 @@ ACCEL_LLAMA_API int accel_llama_logit_max_abs(AccelLlama* model, const float* re
 /* Uncounted read of the logit row (no reference counterpart; for tests). */
 ACCEL_LLAMA_API int accel_llama_logits(AccelLlama* model, float* out, int32_t count);
 /* No reference counterpart (a test seam) for a one-row (decode) forward. enable is a bit
- * mask, default 7. Bit 0: the RMSNorms and SiLU*up run inside the next int8 GEMV (the norm is
+ * mask, default 7. Bit 0: the RMSNorms and SiLU*up run inside the next GEMV (the norm is
  * applied to the product's sums, which rounds differently from normalizing first) instead of
  * as separate kernels. Bit 1: RoPE + KV append, attention and chunk combine run as one kernel
  * instead of three (same bits). Bit 2 (not in exact-products mode; over bit 1): the attention
