@@ -134,7 +134,10 @@ void RunMatmul(const float* a, const AccelHipQuantPlane* aq, const float* b, con
       LaunchExactMatmul(a_f, q8 ? nullptr : b_f, q8 ? view : Q8View{}, c, m, k, n, main, ctx.stream);
     } else if (q8 && m <= 16) {
       if (GemvWantsGroups(m, k, n, view)) view.grouped = StagedGroupTiles(view.q, k, n, ctx.stream, stage_weights);
-      else if (GemvWantsTiles(m, k, n, view)) view.tiled = StagedColumnTiles(view.q, k, n, ctx.stream, stage_weights);
+      else if (GemvWantsTiles(m, k, n, view)) {
+        const bool in_place = Capturing() && GemvTilesOptional(m, k, n, view);
+        view.tiled = StagedColumnTiles(view.q, k, n, ctx.stream, stage_weights && !in_place);
+      }
       LaunchGemvQ8(a_f, view, c, m, k, n, main, ctx.stream);
     } else {
       if (q8 && GemmWantsBf16Image(m, k, n, view)) view.bf16 = StagedBf16Image(view.q, k, n, ctx.stream, stage_weights);
@@ -243,8 +246,7 @@ ACCEL_HIP_API int accel_hip_prepare_quantized(const AccelHipQuantPlane* b_quant,
         Fail(ACCEL_HIP_INVALID_ARGUMENT, "prepare: this plane's scale coordinates fit no staged form (it is dequantized per call)");
       return;
     }
-    const bool groups_ok = k % kGemvGroupRows == 0 && view.zero == nullptr &&
-                           (view.mode == kScalePerCol || view.mode == kScaleConst);
+    const bool groups_ok = GemvGroupForm(k, view);
     const bool bf16_ok = GemmBf16Stageable(k, n, view);
     const bool small_ok = GemmSmallStageable(k, n, view);
     const uint32_t want = layouts != 0 ? layouts

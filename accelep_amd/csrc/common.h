@@ -227,8 +227,15 @@ bool GemmBf16Stageable(int64_t k, int64_t n, const Q8View& v);
 // points or per-row scale, a large matrix; or from the 8-column tiles (m <= 4, the larger m only
 // while the matrix is small). Otherwise W is read in place.
 constexpr int64_t kGemvGroupMinM = 3;
+// Whether the plane can have the group-interleaved copy at all.
+bool GemvGroupForm(int64_t k, const Q8View& v);
 bool GemvWantsGroups(int64_t m, int64_t k, int64_t n, const Q8View& v);
 bool GemvWantsTiles(int64_t m, int64_t k, int64_t n, const Q8View& v);
+// Whether a product that wants tiles and finds none inside a capture reads W in place there: three
+// or four rows of a plane whose group grid fills the CUs. A use of such a weight with more rows stages
+// nothing and is all the preparation a capture needs; other planes' tiles are built by a use of the
+// same rows or by accel_hip_prepare_quantized.
+bool GemvTilesOptional(int64_t m, int64_t k, int64_t n, const Q8View& v);
 
 struct Epilogue {
   float alpha = 1.f;

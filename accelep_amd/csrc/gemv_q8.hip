@@ -1155,12 +1155,12 @@ int64_t CuCount() {
 // better (2048 x 14336 10.6, 11.3 and 11.2, 12.0; 4096 x 14336 15.6, 16.6 and 16.9, 17.7).
 constexpr int64_t kGroupMinElems = int64_t(28) << 20;
 
-bool GroupForm(int64_t k, const Q8View& v) {
+bool GemvGroupForm(int64_t k, const Q8View& v) {
   return k % kGemvGroupRows == 0 && v.zero == nullptr && (v.mode == kScalePerCol || v.mode == kScaleConst);
 }
 
 bool GemvWantsGroups(int64_t m, int64_t k, int64_t n, const Q8View& v) {
-  return m >= kGemvGroupMinM && m <= 16 && k * n >= kGroupMinElems && GroupForm(k, v);
+  return m >= kGemvGroupMinM && m <= 16 && k * n >= kGroupMinElems && GemvGroupForm(k, v);
 }
 
 // The narrow kernel's VALU work grows with m: three or four rows take it only while W is small
@@ -1169,7 +1169,14 @@ bool GemvWantsGroups(int64_t m, int64_t k, int64_t n, const Q8View& v) {
 // groups' form goes in place from 20 Mi elements (4096 x 6144 9.8 us in place, 3072 x 8192 8.9).
 bool GemvWantsTiles(int64_t m, int64_t k, int64_t n, const Q8View& v) {
   if (m <= 2) return true;
-  return m <= 4 && k * n < (GroupForm(k, v) ? int64_t(20) << 20 : kGroupMinElems);
+  return m <= 4 && k * n < (GemvGroupForm(k, v) ? int64_t(20) << 20 : kGroupMinElems);
+}
+
+bool GemvTilesOptional(int64_t m, int64_t k, int64_t n, const Q8View& v) {
+  if (m < kGemvGroupMinM || !GemvGroupForm(k, v)) return false;
+  int64_t groups = 0, splits = 0;
+  SplitBf16Grid(k, n, CuCount(), &groups, &splits);
+  return groups * splits >= CuCount();
 }
 
 bool GemvWaveTileApplies(int64_t m, int64_t k, int64_t n) {
