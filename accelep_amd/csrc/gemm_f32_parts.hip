@@ -19,8 +19,14 @@
 // of bf16 products, what a large bf16 library product reaches (1160 to 1290); 181 us with the
 // compiler's own order of a chunk. 2000 x 1023 x 2047: 136 -> 54 us; 333 x 2048 x 3000: 109 -> 38; 100
 // x 777 x 1001: 19.9 -> 10.4. Error against float64 at k = 4096: 1.15e-6 -> 2.7e-7.
-//  * Tiles whose sums the parts cannot hold (infinities, NaN, the last binade below the fp32
-//    limit, sums below 2^-64) are summed again on the fp32 matrix cores.
+//  * The parts carry an operand whole from 2^-110 up to the last binade below the fp32 limit; of a
+//    smaller one up to 2^-134 is lost. A wave sums its tile again on the fp32 matrix cores where that
+//    shows: a sum that is not finite, or not zero and below 2^-64. Two more cases need a look at the
+//    operands: an operand of 2^32 or more (times the loss it can reach larger sums; without one, a sum of
+//    2^-64 or more loses at most k 2^-102, k 2^-38 of it) and a sum of zero (all of its products may be
+//    lost). There the workgroup reads its operands again, and the tile is summed again if one of them
+//    is not zero and below 2^-110. Following the largest operand takes a thread 8 instructions a chunk (176
+//    us beside 174.6 without, 187 with the lowest exponent followed too); the second reading, 27 us.
 #include "device_common.h"
 
 #include <algorithm>
@@ -75,21 +81,32 @@ __device__ __forceinline__ void LoadRaw(const float* a, const float* b, int64_t 
   for (int t = 0; t < 8; ++t) r.b[t] = b[t * n];
 }
 
+// Operands of this size and more may lift what the parts lose of a tiny one over 2^-64.
+constexpr float kHuge = 0x1p32f;
+
+// largest = max(largest, |x0|, |x1|) in one instruction (NaNs, which the sums show, are left out).
+__device__ __forceinline__ void KeepLargest(float& largest, float x0, float x1) {
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(largest) : "v"(x0), "v"(x1));
+}
+
 // Eight floats (k ascending) to the pieces of the three planes.
 template <int BM>
-__device__ __forceinline__ void StoreParts(u32x4* planes, int piece, const float (&x)[8]) {
+__device__ __forceinline__ void StoreParts(u32x4* planes, int piece, const float (&x)[8], float& largest) {
   uint32_t w[3][4];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) SplitBf16Pair(x[2 * v], x[2 * v + 1], w[0][v], w[1][v], w[2][v]);
+  for (int v = 0; v < 4; ++v) {
+    SplitBf16Pair(x[2 * v], x[2 * v + 1], w[0][v], w[1][v], w[2][v]);
+    KeepLargest(largest, x[2 * v], x[2 * v + 1]);
+  }
 #pragma unroll
   for (int q = 0; q < 3; ++q) planes[q * Shape<BM>::kPlaneVecs + piece] = u32x4{w[q][0], w[q][1], w[q][2], w[q][3]};
 }
 
 template <int BM>
-__device__ __forceinline__ void StoreRaw(u32x4* buf, int a_piece, int b_piece, const Raw& r) {
+__device__ __forceinline__ void StoreRaw(u32x4* buf, int a_piece, int b_piece, const Raw& r, float& largest) {
   const float xa[8] = {r.a[0][0], r.a[0][1], r.a[0][2], r.a[0][3], r.a[1][0], r.a[1][1], r.a[1][2], r.a[1][3]};
-  StoreParts<BM>(buf, a_piece, xa);
-  StoreParts<BM>(buf + 3 * Shape<BM>::kPlaneVecs, b_piece, r.b);
+  StoreParts<BM>(buf, a_piece, xa, largest);
+  StoreParts<BM>(buf + 3 * Shape<BM>::kPlaneVecs, b_piece, r.b, largest);
 }
 
 __device__ __forceinline__ v16f Mfma(const u32x4& a, const u32x4& b, const v16f& c) {
@@ -124,6 +141,22 @@ __device__ __forceinline__ void MultiplyStep(const u32x4* buf, int lane, int wm,
         v16f& acc = q == 0 ? hh[i][j] : cross[i][j];
         acc = Mfma(av[i][kPa[q]], bv[j][kPb[q]], acc);
       }
+}
+
+// Whether some operand that the thread splits in chunks [c0, c1) is not zero and below 2^-110.
+__device__ bool TinyOperand(const float* asrc, const float* bsrc, int64_t n, int64_t c0, int64_t c1, int pad) {
+  uint32_t low = 0xffffffffu;  // of the bits without the sign, less 1
+#pragma unroll 4
+  for (int64_t ch = c0; ch < c1; ++ch) {
+    Raw r;
+    LoadRaw(asrc + ChunkK(ch, pad), bsrc + ChunkK(ch, pad) * n, n, r);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      low = min(low, (__float_as_uint(r.a[e >> 2][e & 3]) << 1) - 1);
+      low = min(low, (__float_as_uint(r.b[e]) << 1) - 1);
+    }
+  }
+  return low < (uint32_t(127 - 110) << 24) - 1;
 }
 
 // The wave's sums over its k of chunks [c0, c1) on v_mfma_f32_32x32x2f32, operands straight from
@@ -222,7 +255,8 @@ GemmF32PartsKernel(PartsArgs p) {
     for (int e = 0; e < 8; ++e)
       if (8 * ag + e >= kBK - pad) raw[0].a[e >> 2][e & 3] = 0.f;
   }
-  StoreRaw<BM>(lds, a_piece, b_piece, raw[0]);
+  float largest = 0.f;  // of the operands this thread splits, without the sign
+  StoreRaw<BM>(lds, a_piece, b_piece, raw[0], largest);
   __syncthreads();
   for (int base = 0; base < chunks; base += 2) {
 #pragma unroll
@@ -239,7 +273,7 @@ GemmF32PartsKernel(PartsArgs p) {
         MultiplyStep<BM>(buf, lane, wm, wn, 0, hh, cross);
         MultiplyStep<BM>(buf, lane, wm, wn, 2, hh, cross);
       }
-      StoreRaw<BM>(lds + ((ch + 1) & 1) * Shape<BM>::kBufVecs, a_piece, b_piece, raw[st ^ 1]);
+      StoreRaw<BM>(lds + ((ch + 1) & 1) * Shape<BM>::kBufVecs, a_piece, b_piece, raw[st ^ 1], largest);
       if constexpr (kGroups == 2) {
         // The operand reads first, then one MFMA, a share of the split and of its stores in turn.
         __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);  // LDS read
@@ -254,7 +288,7 @@ GemmF32PartsKernel(PartsArgs p) {
     }
   }
 
-  uint32_t largest = 0, smallest = 0xffffffffu;  // of the bits without the sign; a zero counts as largest
+  uint32_t top = 0, low = 0xffffffffu, zero = 0;  // of the sums' bits without the sign (less 1: a zero is above all)
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
@@ -263,11 +297,17 @@ GemmF32PartsKernel(PartsArgs p) {
       for (int r = 0; r < 16; ++r) {
         hh[i][j][r] = hh[i][j][r] + cross[i][j][r];
         const uint32_t u = __float_as_uint(hh[i][j][r]) << 1;
-        largest = max(largest, u);
-        smallest = min(smallest, u - 1);
+        top = max(top, u);
+        low = min(low, u - 1);
+        zero = max(zero, u - 1);
       }
-  if (__any(largest >= 0xff000000u || smallest < (uint32_t(127 - 64) << 24) - 1))
-    PlainSums<BM>(p, m0, n0, c0, c0 + chunks, pad, lane, wm, wn, kg, hh);
+  bool again = top >= 0xff000000u || low < (uint32_t(127 - 64) << 24) - 1;
+  const bool huge = __syncthreads_or(largest >= kHuge);
+  if (__syncthreads_or(huge || zero == 0xffffffffu)) {
+    const bool tiny = __syncthreads_or(TinyOperand(asrc, bsrc, p.n, c0, c0 + chunks, pad));
+    again |= tiny && (huge || zero == 0xffffffffu);
+  }
+  if (__any(again)) PlainSums<BM>(p, m0, n0, c0, c0 + chunks, pad, lane, wm, wn, kg, hh);
 
   // Two waves hold a 64 x 64 tile's sums over the two halves of each chunk: wave kg finishes column
   // tile kg and gives its sums of the other one away through LDS.

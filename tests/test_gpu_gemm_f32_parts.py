@@ -70,3 +70,49 @@ def test_gemm_f32_parts_values_beyond_the_bf16_parts(m, k, n):
     same_bits(got[rest, 7], np.where(a[rest, 20] > 0, -np.inf, np.inf).astype(np.float32))
     up = np.float64(2.0 ** 100)  # exact scaling, so the bound's absolute term does not hide the row
     assert_gamma_bound(got[[41]][:, cols].astype(np.float64) * up, a[[41]].astype(np.float64) * up, b[:, cols])
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 101, 75), (1100, 101, 4100)])
+@pytest.mark.parametrize("tiny,huge", [(-118, 60), (-126, 70), (-136, 100), (-145, 20), (-145, 127)])
+def test_gemm_f32_parts_values_below_the_parts(m, k, n, tiny, huge):
+    """Values of 2^tiny (some or all bits below what the parts hold) in a row of A and a column of B
+    against values of 2^huge in the other operand: within the bound of the exact product."""
+    r = np.random.default_rng(1000 + tiny * 7 + huge)
+
+    def values(count, exponent):
+        return np.ldexp(r.uniform(1, 2, count) * r.choice([-1, 1], count), exponent).astype(np.float32)
+
+    a = r.standard_normal((m, k)).astype(np.float32)
+    b = (r.standard_normal((k, n)) * 0.05).astype(np.float32)
+    a[5], b[:, 9] = values(k, tiny), values(k, huge)
+    a[66], b[:, 70] = values(k, huge), values(k, tiny)
+    a[66, 30:] = 0  # the sums stay below the fp32 limit
+    b[30:, 9] = 0
+    got = run(a, b).astype(np.float64)
+    # Scaled (exactly) so that the bound's absolute term, 1e-30 > 2^-100, is k roundings of subnormal
+    # products, 2^-150 each, and hides no more.
+    up = np.float64(2.0 ** 43)
+    rest = [i for i in range(m) if i not in (5, 66)]
+    cols = [j for j in range(n) if j not in (9, 70)]
+    for i, j in (([5], [9]), ([66], [70]), ([5], cols), (rest, [70]), (rest, cols)):
+        assert_gamma_bound(got[np.ix_(i, j)] * up, a[i].astype(np.float64) * up, b[:, j])
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 101, 75), (1100, 101, 4100)])
+@pytest.mark.parametrize("tiny,huge", [(-116, 56), (-122, 66), (-126, 70), (-130, 100)])
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_gemm_f32_parts_tiny_operand_against_huge_ones(m, k, n, tiny, huge, side):
+    """A row of A (a column of B) whose low bits the parts lose, where no sum is small: the other
+    operand is of 2^huge throughout."""
+    r = np.random.default_rng(1000 + tiny * 7 + huge)
+
+    def values(shape, exponent):
+        return np.ldexp(r.uniform(1, 2, shape) * r.choice([-1, 1], shape), exponent).astype(np.float32)
+
+    a = values((m, k), 0 if side == "a" else huge)
+    b = values((k, n), huge if side == "a" else 0)
+    if side == "a":
+        a[60] = values(k, tiny)
+    else:
+        b[:, 60] = values(k, tiny)
+    assert_gamma_bound(run(a, b), a, b)
