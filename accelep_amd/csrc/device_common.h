@@ -33,6 +33,32 @@ __device__ __forceinline__ void SplitBf16Pair(float x0, float x1, uint32_t& hi, 
   lo = PackBf16(r0 - Bf16Low(mid), r1 - Bf16High(mid));
 }
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// acc = the sums of a wave's 32 x 32 tile over `groups` groups of 16 k on v_mfma_f32_32x32x2f32, each
+// operand straight from memory: what the bf16-part kernels fall back to for values that the parts
+// cannot hold. load(g, x, y) brings the lane's 8 values of A row lane % 32 and of B column lane % 32
+// at k 8 * (lane / 32) .. + 7 of group g. Four groups are requested at once: their latency is the cost.
+template <typename Load>
+__device__ __forceinline__ void PlainTileSums(int groups, Load load, f32x16& acc) {
+  constexpr int kAhead = 4;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll 1
+  for (int g0 = 0; g0 < groups; g0 += kAhead) {
+    float x[kAhead][8], y[kAhead][8];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) load(min(g0 + q, groups - 1), x[q], y[q]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      if (g0 + q >= groups) break;  // uniform
+#pragma unroll
+      for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[q][s], y[q][s], acc, 0, 0, 0);
+    }
+  }
+}
+
 // Bias index of element (i, j) for a bias of rank 0..2 right-aligned against [m, n];
 // a dimension of size 1 broadcasts (BiasOffset, src/sim_device.cc:104-124).
 __device__ __forceinline__ int64_t BiasIndex(const Epilogue& e, int64_t i, int64_t j) {

@@ -20,13 +20,15 @@
 // compiler's own order of a chunk. 2000 x 1023 x 2047: 136 -> 54 us; 333 x 2048 x 3000: 109 -> 38; 100
 // x 777 x 1001: 19.9 -> 10.4. Error against float64 at k = 4096: 1.15e-6 -> 2.7e-7.
 //  * The parts carry an operand whole from 2^-110 up to the last binade below the fp32 limit; of a
-//    smaller one up to 2^-134 is lost. A wave sums its tile again on the fp32 matrix cores where that
-//    shows: a sum that is not finite, or not zero and below 2^-64. Two more cases need a look at the
-//    operands: an operand of 2^32 or more (times the loss it can reach larger sums; without one, a sum of
-//    2^-64 or more loses at most k 2^-102, k 2^-38 of it) and a sum of zero (all of its products may be
-//    lost). There the workgroup reads its operands again, and the tile is summed again if one of them
-//    is not zero and below 2^-110. Following the largest operand takes a thread 8 instructions a chunk (176
-//    us beside 174.6 without, 187 with the lowest exponent followed too); the second reading, 27 us.
+//    smaller one up to 2^-134 is lost. A wave sums a 32 x 32 tile again on the fp32 matrix cores where
+//    a sum is not finite, or not zero and below 2^-110. Two more cases need a look at the operands: a
+//    sum of zero (all of its products may be lost) or below 2^-64, and an operand of 2^32 or more (times
+//    the loss it can reach larger sums; without one, a sum of 2^-64 or more loses at most k 2^-102,
+//    k 2^-38 of it). There the workgroup reads its operands again, and the tile is summed again if one
+//    of them is not zero and below 2^-110. 1000 x 4096 x 4096: following the largest operand takes 1.4
+//    us (187 us with the lowest exponent followed too), the second reading 27 us, one infinity in A 104,
+//    a row of 1e-37 204 (349 us in all on the fp32 matrix cores alone; 64 x 64 tiles summed again one k
+//    pair after the other: 440 and 620).
 #include "device_common.h"
 
 #include <algorithm>
@@ -159,44 +161,25 @@ __device__ bool TinyOperand(const float* asrc, const float* bsrc, int64_t n, int
   return low < (uint32_t(127 - 110) << 24) - 1;
 }
 
-// The wave's sums over its k of chunks [c0, c1) on v_mfma_f32_32x32x2f32, operands straight from
-// memory (a dword load per operand, so slow).
+// A 32 x 32 tile's sums over the wave's k of chunks [c0, c1) in plain fp32: rows from m0, columns from n0.
 template <int BM>
-__device__ void PlainSums(const PartsArgs& p, int64_t m0, int64_t n0, int64_t c0, int64_t c1, int pad, int lane, int wm,
-                          int wn, int kg, v16f (&acc)[Shape<BM>::kS][Shape<BM>::kS]) {
-  constexpr int S = Shape<BM>::kS;
-  constexpr int kSpan = kBK / Shape<BM>::kGroups;
-  const float* arow[S];
-  const float* bcol[S];
+__device__ void PlainSums(const PartsArgs& p, int64_t m0, int64_t n0, int64_t c0, int64_t c1, int pad, int lane, int kg,
+                          v16f& acc) {
+  constexpr int kPer = 2 / Shape<BM>::kGroups;  // groups of 16 k of a chunk
+  const float* arow = p.a + min(m0 + (lane & 31), p.m - 1) * p.k;
+  const float* bcol = p.b + min(n0 + (lane & 31), p.n - 1);
+  PlainTileSums(static_cast<int>(c1 - c0) * kPer, [&](int g, float (&x)[8], float (&y)[8]) {
+    const int64_t ch = c0 + g / kPer;
+    const int kl = 16 * (kPer == 1 ? kg : g % kPer) + 8 * (lane >> 5);
+    const int64_t gk = ChunkK(ch, pad) + kl;
+    __builtin_memcpy(x, arow + gk, sizeof(x));
 #pragma unroll
-  for (int i = 0; i < S; ++i) {
-    arow[i] = p.a + min(m0 + (wm * S + i) * 32 + (lane & 31), p.m - 1) * p.k;
-    bcol[i] = p.b + min(n0 + (wn * S + i) * 32 + (lane & 31), p.n - 1);
+    for (int s = 0; s < 8; ++s) y[s] = bcol[(gk + s) * p.n];
+    if (ch != 0) return;
 #pragma unroll
-    for (int j = 0; j < S; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  }
-#pragma unroll 1
-  for (int64_t ch = c0; ch < c1; ++ch) {
-    const int keep = ch == 0 ? kBK - pad : kBK;
-#pragma unroll 1
-    for (int kk = kSpan * kg; kk < kSpan * (kg + 1); kk += 2) {
-      const int kl = kk + (lane >> 5);
-      const bool in = kl < keep;
-      const int64_t gk = ChunkK(ch, pad) + (in ? kl : 0);
-      float av[S], bv[S];
-#pragma unroll
-      for (int i = 0; i < S; ++i) {
-        av[i] = in ? arow[i][gk] : 0.f;
-        bv[i] = in ? bcol[i][gk * p.n] : 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < S; ++i)
-#pragma unroll
-        for (int j = 0; j < S; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-    }
-  }
+    for (int s = 0; s < 8; ++s)
+      if (kl + s >= kBK - pad) x[s] = y[s] = 0.f;
+  }, acc);
 }
 
 template <int BM>
@@ -288,26 +271,35 @@ GemmF32PartsKernel(PartsArgs p) {
     }
   }
 
-  uint32_t top = 0, low = 0xffffffffu, zero = 0;  // of the sums' bits without the sign (less 1: a zero is above all)
+  // Of a tile's sums in this lane: not finite, or not zero and below 2^-110; zero or below 2^-64.
+  bool bad[S][S], small[S][S], any_small = false;
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < S; ++j)
+    for (int j = 0; j < S; ++j) {
+      uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         hh[i][j][r] = hh[i][j][r] + cross[i][j][r];
         const uint32_t u = __float_as_uint(hh[i][j][r]) << 1;
         top = max(top, u);
-        low = min(low, u - 1);
-        zero = max(zero, u - 1);
+        low = min(low, u);
+        low_nonzero = min(low_nonzero, u - 1);
       }
-  bool again = top >= 0xff000000u || low < (uint32_t(127 - 64) << 24) - 1;
+      bad[i][j] = top >= 0xff000000u || low_nonzero < (uint32_t(127 - 110) << 24) - 1;
+      small[i][j] = low < uint32_t(127 - 64) << 24;
+      any_small |= small[i][j];
+    }
   const bool huge = __syncthreads_or(largest >= kHuge);
-  if (__syncthreads_or(huge || zero == 0xffffffffu)) {
-    const bool tiny = __syncthreads_or(TinyOperand(asrc, bsrc, p.n, c0, c0 + chunks, pad));
-    again |= tiny && (huge || zero == 0xffffffffu);
-  }
-  if (__any(again)) PlainSums<BM>(p, m0, n0, c0, c0 + chunks, pad, lane, wm, wn, kg, hh);
+  bool tiny = false;
+  if (__syncthreads_or(huge || any_small))
+    tiny = __syncthreads_or(TinyOperand(asrc, bsrc, p.n, c0, c0 + chunks, pad));
+#pragma unroll
+  for (int i = 0; i < S; ++i)
+#pragma unroll
+    for (int j = 0; j < S; ++j)
+      if (__any(bad[i][j] || (tiny && (huge || small[i][j]))))
+        PlainSums<BM>(p, m0 + (wm * S + i) * 32, n0 + (wn * S + j) * 32, c0, c0 + chunks, pad, lane, kg, hh[i][j]);
 
   // Two waves hold a 64 x 64 tile's sums over the two halves of each chunk: wave kg finishes column
   // tile kg and gives its sums of the other one away through LDS.

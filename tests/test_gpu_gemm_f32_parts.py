@@ -73,7 +73,7 @@ def test_gemm_f32_parts_values_beyond_the_bf16_parts(m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(70, 101, 75), (1100, 101, 4100)])
-@pytest.mark.parametrize("tiny,huge", [(-118, 60), (-126, 70), (-136, 100), (-145, 20), (-145, 127)])
+@pytest.mark.parametrize("tiny,huge", [(-118, 60), (-126, 70), (-136, 100), (-145, 20), (-145, 127), (-70, -70)])
 def test_gemm_f32_parts_values_below_the_parts(m, k, n, tiny, huge):
     """Values of 2^tiny (some or all bits below what the parts hold) in a row of A and a column of B
     against values of 2^huge in the other operand: within the bound of the exact product."""
