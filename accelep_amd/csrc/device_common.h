@@ -37,24 +37,26 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // acc = the sums of a wave's 32 x 32 tile over `groups` groups of 16 k on v_mfma_f32_32x32x2f32, each
 // operand straight from memory: what the bf16-part kernels fall back to for values that the parts
-// cannot hold. load(g, x, y) brings the lane's 8 values of A row lane % 32 and of B column lane % 32
-// at k 8 * (lane / 32) .. + 7 of group g. Four groups are requested at once: their latency is the cost.
-template <typename Load>
-__device__ __forceinline__ void PlainTileSums(int groups, Load load, f32x16& acc) {
-  constexpr int kAhead = 4;
+// cannot hold. load(g, raw) requests what the lane needs of group g and use(g, raw, x, y) makes its 8
+// values of A row lane % 32 and of B column lane % 32 of it, at k 8 * (lane / 32) .. + 7. kAhead groups
+// are requested at once: their latency is the cost.
+template <typename Raw, int kAhead, typename Load, typename Use>
+__device__ __forceinline__ void PlainTileSums(int groups, Load load, Use use, f32x16& acc) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 #pragma unroll 1
   for (int g0 = 0; g0 < groups; g0 += kAhead) {
-    float x[kAhead][8], y[kAhead][8];
+    Raw raw[kAhead];
 #pragma unroll
-    for (int q = 0; q < kAhead; ++q) load(min(g0 + q, groups - 1), x[q], y[q]);
+    for (int q = 0; q < kAhead; ++q) load(min(g0 + q, groups - 1), raw[q]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) {
       if (g0 + q >= groups) break;  // uniform
+      float x[8], y[8];
+      use(g0 + q, raw[q], x, y);
 #pragma unroll
-      for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[q][s], y[q][s], acc, 0, 0, 0);
+      for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], acc, 0, 0, 0);
     }
   }
 }

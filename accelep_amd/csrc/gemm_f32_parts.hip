@@ -168,18 +168,23 @@ __device__ void PlainSums(const PartsArgs& p, int64_t m0, int64_t n0, int64_t c0
   constexpr int kPer = 2 / Shape<BM>::kGroups;  // groups of 16 k of a chunk
   const float* arow = p.a + min(m0 + (lane & 31), p.m - 1) * p.k;
   const float* bcol = p.b + min(n0 + (lane & 31), p.n - 1);
-  PlainTileSums(static_cast<int>(c1 - c0) * kPer, [&](int g, float (&x)[8], float (&y)[8]) {
-    const int64_t ch = c0 + g / kPer;
-    const int kl = 16 * (kPer == 1 ? kg : g % kPer) + 8 * (lane >> 5);
-    const int64_t gk = ChunkK(ch, pad) + kl;
-    __builtin_memcpy(x, arow + gk, sizeof(x));
+  const auto first_k = [&](int g) { return 16 * (kPer == 1 ? kg : g % kPer) + 8 * (lane >> 5); };
+  PlainTileSums<Raw, 4>(
+      static_cast<int>(c1 - c0) * kPer,
+      [&](int g, Raw& r) {
+        const int64_t gk = ChunkK(c0 + g / kPer, pad) + first_k(g);
+        LoadRaw(arow + gk, bcol + gk * p.n, p.n, r);
+      },
+      [&](int g, const Raw& r, float (&x)[8], float (&y)[8]) {
+        const int keep = c0 + g / kPer == 0 ? kBK - pad : kBK;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) y[s] = bcol[(gk + s) * p.n];
-    if (ch != 0) return;
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-      if (kl + s >= kBK - pad) x[s] = y[s] = 0.f;
-  }, acc);
+        for (int s = 0; s < 8; ++s) {
+          const bool in = first_k(g) + s < keep;
+          x[s] = in ? r.a[s >> 2][s & 3] : 0.f;
+          y[s] = in ? r.b[s] : 0.f;
+        }
+      },
+      acc);
 }
 
 template <int BM>

@@ -37,6 +37,10 @@
 //    333 x 4096 x 4096 with zero points 223 us (50 TFLOP/s) -> 55, with a per-row scale 227 -> 56,
 //    333 x 4095 x 4097 440 -> 77, 2000 x 2047 x 14335 1651 -> 407, 2000 x 2048 x 14336 with zero
 //    points 1011 -> 383. Error against float64 at k = 4096: 1.1e-6 -> 1.1e-7 .. 2.5e-7.
+//  * Values that the parts cannot hold (infinities, NaN, the last binade below the fp32 limit, sums
+//    below 2^-64) have the general forms sum their 32 x 32 tile again on the fp32 matrix cores. 2000 x
+//    2048 x 14336 with zero points and one infinity 1008 us (2731 with 64 x 64 tiles, one k pair after
+//    the other; 1003 on the fp32 matrix cores alone), 333 x 4096 x 4096 102 (285; 222).
 #include "device_common.h"
 
 #include <algorithm>
@@ -269,67 +273,53 @@ __device__ __forceinline__ void ComputeChunk(const uint32_t* buf, int lane, int 
   }
 }
 
-// The wave's raw sums over k [kb, ke) on v_mfma_f32_32x32x2f32 with both operands straight from
-// memory: for tiles whose values the bf16 parts cannot hold (infinities, NaN, the last binade
-// below the fp32 limit, or values so small that the parts leave the normal range). Slow (a dword
-// load per operand), and only such tiles take it.
-template <int BM>
-__device__ void PlainSums(const Q8GemmArgs& p, int64_t m0, int64_t n0, int64_t kb, int64_t ke, int lane, int wm, int wn,
-                          v16f (&acc)[Tile<BM>::kS][Tile<BM>::kS]) {
-  constexpr int S = Tile<BM>::kS;
-  const float* arow[S];
-  int64_t col[S];
-  float zc[S];
-#pragma unroll
-  for (int i = 0; i < S; ++i) {
-    arow[i] = p.a + min(m0 + wm * (BM / 2) + i * 32 + (lane & 31), p.m - 1) * p.k;
-    col[i] = min(n0 + wn * (BM / 2) + i * 32 + (lane & 31), p.n - 1);
-    zc[i] = p.zero != nullptr && p.mode != kScalePerRow
-                ? static_cast<float>(p.zero[p.mode == kScalePerCol ? col[i] : p.const_index]) : 0.f;
-#pragma unroll
-    for (int j = 0; j < S; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  }
-#pragma unroll 1
-  for (int64_t kk = kb; kk < ke; kk += 2) {
-    const int64_t gk = min(kk + (lane >> 5), ke - 1);
-    const bool in = kk + (lane >> 5) < ke;
-    float rs = 1.f, rz = 0.f;
-    if (p.mode == kScalePerRow) {
-      rs = p.scale[gk];
-      if (p.zero != nullptr) rz = static_cast<float>(p.zero[gk]);
-    }
-    float av[S], bv[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) {
-      av[i] = in ? arow[i][gk] : 0.f;
-      const float w = static_cast<float>(p.q[gk * p.n + col[i]]) - zc[i] - rz;
-      bv[i] = in ? __fmul_rn(w, rs) : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < S; ++i)
-#pragma unroll
-      for (int j = 0; j < S; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], bv[j], acc[i][j], 0, 0, 0);
-  }
-}
+// What a lane reads of 16 k for PlainSums: 8 activations, the 8 rows' bytes of its column, and with a
+// per-row scale the rows' scales and zero points.
+template <int kForm>
+struct PlainRaw {
+  v4f a[2];
+  int8_t q[8];
+  float s[kForm == kRows ? 8 : 1];
+  int8_t z[kForm == kRows ? 8 : 1];
+};
 
-// Whether some raw sum of the wave calls for PlainSums: non-finite, or nonzero and so small (below
-// 2^-64) that parts below 2^-110 may have made it.
-template <int S>
-__device__ __forceinline__ bool NeedsPlainSums(const v16f (&acc)[S][S]) {
-  uint32_t largest = 0, smallest = 0xffffffffu;  // of the bits without the sign; a zero counts as largest
+// A 32 x 32 tile's raw sums over chunks [c0, c1) in plain fp32: rows from m0, columns from n0.
+template <int kForm>
+__device__ void PlainSums(const Q8GemmArgs& p, int64_t m0, int64_t n0, int64_t c0, int64_t c1, int pad, int lane,
+                          v16f& acc) {
+  const float* arow = p.a + min(m0 + (lane & 31), p.m - 1) * p.k;
+  const int64_t col = min(n0 + (lane & 31), p.n - 1);
+  float zc = 0.f;
+  if (kForm == kCols && p.zero != nullptr) zc = static_cast<float>(p.zero[p.mode == kScalePerCol ? col : p.const_index]);
+  const auto first_k = [&](int g) { return 16 * (g % 2) + 8 * (lane >> 5); };
+  PlainTileSums<PlainRaw<kForm>, kForm == kRows ? 2 : 4>(
+      static_cast<int>(c1 - c0) * 2,
+      [&](int g, PlainRaw<kForm>& r) {
+        const int64_t gk = ChunkK<kForm>(c0 + g / 2, pad) + first_k(g);
+        r.a[0] = LoadAny<v4f>(arow + gk);
+        r.a[1] = LoadAny<v4f>(arow + gk + 4);
 #pragma unroll
-  for (int i = 0; i < S; ++i)
+        for (int s = 0; s < 8; ++s) r.q[s] = p.q[(gk + s) * p.n + col];
+        if constexpr (kForm == kRows) {
 #pragma unroll
-    for (int j = 0; j < S; ++j)
+          for (int s = 0; s < 8; ++s) {
+            r.s[s] = p.scale[gk + s];
+            r.z[s] = p.zero != nullptr ? p.zero[gk + s] : 0;
+          }
+        }
+      },
+      [&](int g, const PlainRaw<kForm>& r, float (&x)[8], float (&y)[8]) {
+        const int keep = c0 + g / 2 == 0 ? kBK - pad : kBK;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
-        largest = max(largest, u);
-        smallest = min(smallest, u - 1);
-      }
-  return __any(largest >= 0xff000000u || smallest < (uint32_t(127 - 64) << 24) - 1);
+        for (int s = 0; s < 8; ++s) {
+          const bool in = first_k(g) + s < keep;
+          float w = static_cast<float>(r.q[s]) - zc;
+          if constexpr (kForm == kRows) w = __fmul_rn(w - static_cast<float>(r.z[s]), r.s[s]);
+          x[s] = in ? r.a[s >> 2][s & 3] : 0.f;
+          y[s] = in ? w : 0.f;
+        }
+      },
+      acc);
 }
 
 template <int BM, int kForm>
@@ -412,16 +402,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
     }
   }
 
+  uint32_t bad = 0;  // the tiles (bit i * S + j) with a sum in this lane that is not finite, or not zero and below 2^-64
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < S; ++j)
+    for (int j = 0; j < S; ++j) {
+      uint32_t top = 0, low = 0xffffffffu;  // of the bits without the sign (less 1: a zero is above all)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
-
+      for (int r = 0; r < 16; ++r) {
+        acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
+        const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
+        top = max(top, u);
+        low = min(low, u - 1);
+      }
+      if (top >= 0xff000000u || low < (uint32_t(127 - 64) << 24) - 1) bad |= 1u << (i * S + j);
+    }
   if constexpr (kForm != kPlain) {
-    if (NeedsPlainSums<S>(acc))
-      PlainSums<BM>(p, m0, n0, ChunkK<kForm>(c0, pad), ChunkK<kForm>(c0 + chunks, pad), lane, wm, wn, acc);
+    int tail = lane;
+    asm("" : "+v"(tail));  // addresses made from it are not formed before the loop and kept through it
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int j = 0; j < S; ++j)
+        if (__any((bad >> (i * S + j) & 1u) != 0))
+          PlainSums<kForm>(p, m0 + wm * (BM / 2) + i * 32, n0 + wn * (BM / 2) + j * 32, c0, c0 + chunks, pad, tail,
+                           acc[i][j]);
   }
   // Element r of a 32 x 32 tile sits at row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.
   if (p.partials != nullptr) {  // SplitReduceKernel adds the splits in order, scales, applies the epilogue
