@@ -37,10 +37,13 @@
 //    333 x 4096 x 4096 with zero points 223 us (50 TFLOP/s) -> 55, with a per-row scale 227 -> 56,
 //    333 x 4095 x 4097 440 -> 77, 2000 x 2047 x 14335 1651 -> 407, 2000 x 2048 x 14336 with zero
 //    points 1011 -> 383. Error against float64 at k = 4096: 1.1e-6 -> 1.1e-7 .. 2.5e-7.
-//  * Values that the parts cannot hold (infinities, NaN, the last binade below the fp32 limit, sums
-//    below 2^-64) have the general forms sum their 32 x 32 tile again on the fp32 matrix cores. 2000 x
-//    2048 x 14336 with zero points and one infinity 1008 us (2731 with 64 x 64 tiles, one k pair after
-//    the other; 1003 on the fp32 matrix cores alone), 333 x 4096 x 4096 102 (285; 222).
+//  * The parts carry an activation whole from 2^-110 up to the last binade below the fp32 limit; of
+//    a smaller one up to 2^-134 is lost, which reaches no sum of 2^-64 or more. The general forms sum
+//    a 32 x 32 tile again on the fp32 matrix cores where a sum is not finite, or not zero and below
+//    2^-110, or below 2^-64 (zero too) beside an activation below 2^-110, which the wave looks for in its
+//    rows of A then. 2000 x 2048 x 14336 with zero points: a row of zeros 8 us, one infinity 1008 us in
+//    all (2731 with 64 x 64 tiles, one k pair after the other; 1003 on the fp32 matrix cores alone);
+//    333 x 4096 x 4096: 4 us, 102 us (285; 222).
 #include "device_common.h"
 
 #include <algorithm>
@@ -322,6 +325,43 @@ __device__ void PlainSums(const Q8GemmArgs& p, int64_t m0, int64_t n0, int64_t c
       acc);
 }
 
+// Whether some activation of rows m0 .. m0 + rows - 1 in chunks [c0, c1) is not zero and, times its row
+// scale where there is one, below 2^-110: a lane takes 4 k of every eighth row.
+template <int kForm>
+__device__ bool TinyActivation(const Q8GemmArgs& p, int64_t m0, int rows, int64_t c0, int64_t c1, int pad, int lane) {
+  constexpr int kAhead = 8;
+  const int64_t kb = ChunkK<kForm>(c0, pad), ke = ChunkK<kForm>(c1, pad);
+  uint32_t low = 0xffffffffu;  // of the bits without the sign, less 1
+#pragma unroll 1
+  for (int r = lane >> 3; r < rows; r += 16) {
+    const float* row[2] = {p.a + min(m0 + r, p.m - 1) * p.k, p.a + min(m0 + r + 8, p.m - 1) * p.k};
+#pragma unroll 1
+    for (int64_t k0 = kb + 4 * (lane & 7); k0 < ke; k0 += kAhead * kBK) {
+      v4f x[kAhead][2], s[kAhead];
+#pragma unroll
+      for (int h = 0; h < kAhead; ++h) {
+        const int64_t k1 = min(k0 + h * kBK, ke - 4);
+        x[h][0] = LoadAny<v4f>(row[0] + k1);
+        x[h][1] = LoadAny<v4f>(row[1] + k1);
+        if constexpr (kForm == kRows) s[h] = LoadAny<v4f>(p.scale + k1);
+      }
+#pragma unroll
+      for (int h = 0; h < kAhead; ++h)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const float v = x[h][t >> 2][t & 3];
+          uint32_t u = __float_as_uint(v) << 1;
+          if constexpr (kForm == kRows) {
+            const uint32_t us = __float_as_uint(__fmul_rn(v, s[h][t & 3])) << 1;
+            u = u == 0 || s[h][t & 3] == 0.f ? 0 : max(us, 1u);
+          }
+          low = min(low, u - 1);
+        }
+    }
+  }
+  return low < (uint32_t(127 - 110) << 24) - 1;
+}
+
 template <int BM, int kForm>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 128 ? 2 : 3))) void GemmQ8Bf16Kernel(
     Q8GemmArgs p) {
@@ -402,24 +442,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
     }
   }
 
-  uint32_t bad = 0;  // the tiles (bit i * S + j) with a sum in this lane that is not finite, or not zero and below 2^-64
+  // The tiles (bit i * S + j) with a sum in this lane that is not finite, or not zero and below 2^-110;
+  // those with one below 2^-64, zero too (the columns past n have no weights, so their sums are zero).
+  uint32_t bad = 0, small = 0;
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
     for (int j = 0; j < S; ++j) {
-      uint32_t top = 0, low = 0xffffffffu;  // of the bits without the sign (less 1: a zero is above all)
+      uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
         const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
         top = max(top, u);
-        low = min(low, u - 1);
+        low = min(low, u);
+        low_nonzero = min(low_nonzero, u - 1);
       }
-      if (top >= 0xff000000u || low < (uint32_t(127 - 64) << 24) - 1) bad |= 1u << (i * S + j);
+      if (top >= 0xff000000u || low_nonzero < (uint32_t(127 - 110) << 24) - 1) bad |= 1u << (i * S + j);
+      if (low < uint32_t(127 - 64) << 24 && n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n) small |= 1u << (i * S + j);
     }
   if constexpr (kForm != kPlain) {
     int tail = lane;
     asm("" : "+v"(tail));  // addresses made from it are not formed before the loop and kept through it
+    if (__any(small != 0) &&
+        __any(TinyActivation<kForm>(p, m0 + wm * (BM / 2), BM / 2, c0, c0 + chunks, pad, tail)))
+      bad |= small;
 #pragma unroll
     for (int i = 0; i < S; ++i)
 #pragma unroll

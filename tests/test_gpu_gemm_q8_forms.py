@@ -95,3 +95,21 @@ def test_gemm_q8_forms_values_beyond_the_bf16_parts(mode, zero):
     assert np.isnan(got[17]).all()
     up = np.float64(2.0 ** 100)  # exact scaling, so the bound's absolute term does not hide the row
     assert_gamma_bound(got[[41]].astype(np.float64) * up, a[[41]].astype(np.float64) * up, w)
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 101, 75), (700, 1000, 1100)])
+@pytest.mark.parametrize("mode,zero", FORMS)
+def test_gemm_q8_forms_activations_below_the_parts(m, k, n, mode, zero):
+    """A row whose activations are all below the smallest bf16 gives their product with the weights
+    (2^100 scales, so that the results are far from the fp32 minimum), not zero; zero rows stay zero."""
+    r = np.random.default_rng(6)
+    q, s, z = weight(r, k, n, mode, zero)
+    s *= np.float32(2.0 ** (100 if mode != "row" else 10))
+    a = r.standard_normal((m, k)).astype(np.float32)
+    a[5] = r.integers(1, 16, size=k) * np.float32(2.0 ** -140)
+    a[68] = 0
+    w = dequant(q, s, z, mode).astype(np.float64)
+    got = run(a, q, s, z, mode).astype(np.float64)
+    up = np.float64(2.0 ** 43)  # exact: the bound's absolute term stays below what subnormal sums round
+    assert_gamma_bound(got * up, a.astype(np.float64) * up, w)
+    assert not got[68].any()
