@@ -6,8 +6,14 @@
 //  * q - z is an integer in [-255, 255], which bf16 holds exactly;
 //  * an activation x (times the row's scale where it has one: fl(x * s), one rounding where the
 //    reference rounds (q - z) * s) is the sum of three bf16 parts, which carry its 24 bits.
-// Only the fp32 accumulation rounds. Workgroups whose sums the parts cannot hold (non-finite, or
-// nonzero and below 2^-64) sum again in plain fp32.
+// Only the fp32 accumulation rounds. The parts carry an activation whole from 2^-110 up to the last
+// binade below the fp32 limit; of a smaller one up to 2^-134 is lost, which reaches no sum of 2^-64 or
+// more. A workgroup takes its products again on v_mfma_f32_16x16x4f32 for the rows where a sum is not
+// finite, or not zero and below 2^-110, or below 2^-64 (zero too) beside an activation below 2^-110, which
+// it looks for in those rows then. With zero points, 4096 x 4096, m = 8: 9.6 us, one infinity 16.4, a row of
+// zeros 13.3; 4096 x 14336, m = 16: 19.9, 45.7 and 24.0 (with the elements of a workgroup summed one weight
+// after the other 59 and 1200 us for the infinity). Following the lowest activation in the loop
+// instead of looking for it costs ordinary calls 0.2 to 0.6 us.
 //
 //  * A workgroup owns 16 * V columns over one split of K. Its waves take 32-row blocks in turn;
 //    lane l reads V consecutive bytes (slot l % 16) of rows 8g .. 8g + 7, g = l / 16, of the block,
@@ -138,7 +144,10 @@ __device__ __forceinline__ void LoadTail(const int8_t* qcol, const float* arow, 
     }
     const float x = arow[r];
     t.x[u] = row + u < rows ? x : 0.f;
-    if constexpr (kForm >= kRow) t.s[u] = p.scale[kb + r];
+    if constexpr (kForm >= kRow) {
+      const float sc = p.scale[kb + r];
+      t.s[u] = row + u < rows ? sc : 0.f;
+    }
     if constexpr (kForm == kRowZero) t.z[u] = p.zero[kb + r];
   }
 }
@@ -189,28 +198,68 @@ __device__ __forceinline__ void Multiply(const Block<V, kForm>& t, const float (
                                                       rest[c], 0, 0, 0);
 }
 
-// One element's sum over rows [kb, kb + rows) in plain fp32.
-template <int kForm>
-__device__ float PlainSum(const int8_t* q, const float* arow, const Q8InPlaceArgs& p, int32_t kb, int32_t rows,
-                          int64_t n, int64_t col) {
-  float zc = 0.f;
-  if constexpr (kForm == kZero) zc = static_cast<float>(p.zero[p.mode == kScalePerCol ? col : p.const_index]);
-  float s = 0.f;
-#pragma unroll 1
-  for (int32_t r = kb; r < kb + rows; ++r) {
-    float w = static_cast<float>(q[r * n + col]) - zc;
-    if constexpr (kForm == kRowZero) w -= static_cast<float>(p.zero[r]);
-    if constexpr (kForm >= kRow) w = __fmul_rn(w, p.scale[r]);
-    s = __builtin_fmaf(arow[r], w, s);
-  }
-  return s;
+// The same block in plain fp32: row 8g + u of it is k slot g of MFMA u.
+template <int V, int kForm>
+__device__ __forceinline__ void MultiplyPlain(const Block<V, kForm>& t, const float (&zc)[V], v4f (&acc)[V]) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      float w = ByteToFloat(t.w[u][c >> 2], c & 3);
+      if constexpr (kForm == kZero) w -= zc[c];
+      if constexpr (kForm == kRowZero) w -= static_cast<float>(t.z[u]);
+      if constexpr (kForm >= kRow) w = __fmul_rn(w, t.s[u]);
+      acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.x[u], w, acc[c], 0, 0, 0);
+    }
 }
 
-// Whether a raw sum calls for PlainSum: non-finite, or nonzero and so small (below 2^-64) that
-// parts below 2^-110 may have made it.
-__device__ __forceinline__ bool NeedsPlainSum(float s) {
-  const uint32_t u = __float_as_uint(s) << 1;
-  return u >= 0xff000000u || (u != 0 && u < (uint32_t(127 - 64) << 24));
+// The wave's sums over its blocks of the split in plain fp32, for the group of columns from col0.
+template <int V, int kForm>
+__device__ void PlainSums(const int8_t* q, const float* a, const Q8InPlaceArgs& p, int32_t m, int32_t k, int32_t kb,
+                          int64_t n, int64_t col0, int rows, int wave, int lane, v4f (&acc)[V]) {
+  const int slot = lane & 15, g = lane >> 4;
+  const int64_t col = min(col0 + V * slot, n - V);
+  const int8_t* qcol = q + kb * n + col;
+  const float* arow = a + static_cast<int64_t>(slot < m ? slot : m - 1) * k + kb;
+  float zc[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+    zc[j] = kForm == kZero ? static_cast<float>(p.zero[p.mode == kScalePerCol ? col + j : p.const_index]) : 0.f;
+  }
+  const int whole = rows / kBlockRows;
+  for (int i = wave; i < whole; i += kWaves) {
+    Block<V, kForm> t;
+    LoadBlock<V, kForm>(qcol, arow, p, kb, n, i * kBlockRows + 8 * g, t);
+    MultiplyPlain<V, kForm>(t, zc, acc);
+  }
+  if (rows % kBlockRows != 0 && wave == whole % kWaves) {
+    Block<V, kForm> t;
+    LoadTail<V, kForm>(qcol, arow, p, kb, n, whole * kBlockRows + 8 * g, rows, t);
+    MultiplyPlain<V, kForm>(t, zc, acc);
+  }
+}
+
+// The rows (bit i) of A[m, k] at `a` that hold an activation in this thread's k of [kb, kb + rows) which is
+// not zero and, times its row scale where there is one, below 2^-110.
+template <int kForm>
+__device__ uint32_t TinyRows(const float* a, const Q8InPlaceArgs& p, int32_t m, int32_t k, int32_t kb, int32_t rows,
+                             int tid) {
+  uint32_t tiny = 0;
+#pragma unroll 1
+  for (int r = kb + tid; r < kb + rows; r += 64 * kWaves) {
+    const float s = kForm >= kRow ? p.scale[r] : 1.f;
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = a[static_cast<int64_t>(min(i, m - 1)) * k + r];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      uint32_t u = __float_as_uint(x[i]) << 1;
+      if constexpr (kForm >= kRow) u = u == 0 || s == 0.f ? 0 : max(__float_as_uint(__fmul_rn(x[i], s)) << 1, 1u);
+      if (u - 1 < (uint32_t(127 - 110) << 24) - 1) tiny |= 1u << i;
+    }
+  }
+  return tiny;
 }
 
 // What the first loads need leads the arguments (preloaded into SGPRs at wave launch). Grid: one
@@ -225,11 +274,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(V <
   constexpr int kThreads = 64 * kWaves;
   __shared__ float red[kWaves][16][17 * V];  // column V * slot + j of a group at 17 * j + slot
   __shared__ bool is_last;
+  __shared__ uint32_t again[2];  // rows to sum again; rows with a sum below 2^-64
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int slot = lane & 15;
   const int g = lane >> 4;
+  if (tid == 0) again[0] = again[1] = 0;
   const int per_xcd = static_cast<int>(gridDim.x / kXcds);
   const int pair = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
   if (pair >= pairs) return;
@@ -297,26 +348,46 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(V <
   const int64_t out_col = min(own, n - V) + c % V;
   const bool live_col = out_col >= own && tid / kCols < 16;
   float sum[kPer];
-  bool plain = false;
+  const auto wave_sum = [&](int e) {
+    const int at = 17 * (c % V) + c / V;
+    float s = red[0][i0 + e * kStep][at];
+#pragma unroll
+    for (int v = 1; v < kWaves; ++v) s = s + red[v][i0 + e * kStep][at];
+    return s;
+  };
+  uint32_t bad = 0, small = 0;  // rows of A
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
     const int i = i0 + e * kStep;
-    const int at = 17 * (c % V) + c / V;
-    float s = red[0][i][at];
-#pragma unroll
-    for (int v = 1; v < kWaves; ++v) s = s + red[v][i][at];
-    sum[e] = s;
-    plain |= i < m && NeedsPlainSum(s);
+    sum[e] = wave_sum(e);
+    const uint32_t u = __float_as_uint(sum[e]) << 1;
+    if (!live_col || i >= m) continue;
+    if (u >= 0xff000000u || u - 1 < (uint32_t(127 - 110) << 24) - 1) bad |= 1u << i;
+    if (u < uint32_t(127 - 64) << 24) small |= 1u << i;
   }
-  if (__syncthreads_or(plain)) {
-#pragma unroll 1
-    for (int e = 0; e < kPer; ++e) {
-      const int i = i0 + e * kStep;
-      if (!live_col || i >= m) continue;
-      const float s = PlainSum<kForm>(q, a + static_cast<int64_t>(i) * k, p, kb, rows, n, out_col);
+  if (bad != 0) atomicOr(&again[0], bad);
+  if (small != 0) atomicOr(&again[1], small);
+  __syncthreads();
+  if ((again[0] | again[1]) != 0) {
+    if (again[1] != 0) {
+      const uint32_t tiny = TinyRows<kForm>(a, p, m, k, kb, rows, tid) & again[1];
+      if (tiny != 0) atomicOr(&again[0], tiny);
+      __syncthreads();
+    }
+    const uint32_t redo = again[0];
+    if (redo != 0) {
+      int tail = lane;
+      // addresses made from it are not formed before the loop and kept through it
+      if constexpr (kForm == kRowZero) asm("" : "+v"(tail));
+      PlainSums<V, kForm>(q, a, p, m, k, kb, n, static_cast<int64_t>(group) * kCols, rows, wave, tail, acc);
 #pragma unroll
-      for (int f = 0; f < kPer; ++f)
-        if (f == e) sum[f] = s;
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < V; ++j) red[wave][4 * g + r][17 * j + slot] = acc[j][r];
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < kPer; ++e)
+        if (redo >> (i0 + e * kStep) & 1u) sum[e] = wave_sum(e);
     }
   }
   if (splits > 1) {

@@ -63,6 +63,30 @@ def test_gemv_q8_in_place_values_beyond_the_bf16_parts(mode, zero):
     assert_gamma_bound(got[[6]].astype(np.float64) * up, a[[6]].astype(np.float64) * up, w)
 
 
+@pytest.mark.parametrize("m,k,n", [(7, 33, 2), (9, 1101, 75), (16, 2051, 2049), (13, 2047, 14345)])
+@pytest.mark.parametrize("mode,zero", [("col", False)] + FORMS)
+def test_gemv_q8_in_place_activations_below_the_parts(m, k, n, mode, zero):
+    """A row whose activations are all below the smallest bf16 gives their product with the weights
+    (2^100 scales, so that the results are far from the fp32 minimum), not zero; zero rows stay zero,
+    and an infinite last row scale reaches the rows that have an activation there."""
+    r = np.random.default_rng(6)
+    q, s, z = weight(r, k, n, mode, zero)
+    s *= np.float32(2.0 ** (100 if mode != "row" else 10))
+    a = r.standard_normal((m, k)).astype(np.float32)
+    a[5] = r.integers(1, 16, size=k) * np.float32(2.0 ** -140)
+    a[2] = 0
+    w = dequant(q, s, z, mode).astype(np.float64)
+    got = run(a, q, s, z, mode).astype(np.float64)
+    up = np.float64(2.0 ** 43)  # exact: the bound's absolute term stays below what subnormal sums round
+    assert_gamma_bound(got * up, a.astype(np.float64) * up, w)
+    assert not got[2].any()
+    if mode == "row":
+        s[-1] = np.inf
+        with np.errstate(invalid="ignore"):
+            sign = np.sign(a[:, -1:] * (q[-1].astype(np.float32) - (z[-1].astype(np.float32) if zero else 0)))
+        same_bits(run(a, q, s, z, mode), np.where(sign == 0, np.nan, np.copysign(np.inf, sign)).astype(np.float32))
+
+
 @pytest.mark.parametrize("m,zero", [(8, True), (8, False), (4, False)])
 def test_gemv_q8_in_place_in_a_capture(m, zero):
     """No staged copy is needed: captured before any other use of the weight, replayed with the
