@@ -33,6 +33,18 @@ __device__ __forceinline__ void SplitBf16Pair(float x0, float x1, uint32_t& hi, 
   lo = PackBf16(r0 - Bf16Low(mid), r1 - Bf16High(mid));
 }
 
+// The same for any value: hi and mid stay at or below the largest bf16, so an infinity comes out as
+// finite parts and an infinite lo, a NaN as a NaN lo, and a finite value above the largest bf16 keeps
+// its bits in mid and lo. Products of the parts then sum to what the product of x is.
+__device__ __forceinline__ void SplitBf16PairAny(float x0, float x1, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  constexpr float kMax = 0x1.fep127f;
+  hi = PackBf16(__builtin_amdgcn_fmed3f(x0, -kMax, kMax), __builtin_amdgcn_fmed3f(x1, -kMax, kMax));
+  const float r0 = x0 - Bf16Low(hi);
+  const float r1 = x1 - Bf16High(hi);
+  mid = PackBf16(__builtin_amdgcn_fmed3f(r0, -kMax, kMax), __builtin_amdgcn_fmed3f(r1, -kMax, kMax));
+  lo = PackBf16(r0 - Bf16Low(mid), r1 - Bf16High(mid));
+}
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // acc = the sums of a wave's 32 x 32 tile over `groups` groups of 16 k on v_mfma_f32_32x32x2f32, each

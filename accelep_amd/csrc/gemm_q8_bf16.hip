@@ -43,7 +43,9 @@
 //    2^-110, or below 2^-64 (zero too) beside an activation below 2^-110, which the wave looks for in its
 //    rows of A then. 2000 x 2048 x 14336 with zero points: a row of zeros 8 us, one infinity 1008 us in
 //    all (2731 with 64 x 64 tiles, one k pair after the other; 1003 on the fp32 matrix cores alone);
-//    333 x 4096 x 4096: 4 us, 102 us (285; 222).
+//    333 x 4096 x 4096: 4 us, 102 us (285; 222). The plain form sums a tile again only for sums that
+//    are not finite, and the staged-copy kernels split any activation so that its products come out
+//    as x's do (SplitBf16PairAny): there activations below 2^-134 count as zero.
 #include "device_common.h"
 
 #include <algorithm>
@@ -442,29 +444,44 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
     }
   }
 
-  // The tiles (bit i * S + j) with a sum in this lane that is not finite, or not zero and below 2^-110;
-  // those with one below 2^-64, zero too (the columns past n have no weights, so their sums are zero).
+  // The tiles (bit i * S + j) with a sum in this lane that is not finite and, in the general forms, not
+  // zero and below 2^-110; those with one below 2^-64, zero too (the columns past n have no weights, so
+  // their sums are zero). The plain form adds its sums up first, which shows whether one is not finite:
+  // its K ranges can be short (333 x 1024 x 2048 19.8 us, 21.1 with every sum looked at).
   uint32_t bad = 0, small = 0;
+  float total = 0.f;
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
     for (int j = 0; j < S; ++j) {
-      uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
-        const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
-        top = max(top, u);
-        low = min(low, u);
-        low_nonzero = min(low_nonzero, u - 1);
+        if constexpr (kForm == kPlain) total += acc[i][j][r];
       }
-      if (top >= 0xff000000u || low_nonzero < (uint32_t(127 - 110) << 24) - 1) bad |= 1u << (i * S + j);
-      if (low < uint32_t(127 - 64) << 24 && n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n) small |= 1u << (i * S + j);
     }
-  if constexpr (kForm != kPlain) {
+  if (kForm != kPlain || __any(!(fabsf(total) < INFINITY))) {
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+      for (int j = 0; j < S; ++j) {
+        uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
+          top = max(top, u);
+          low = min(low, u);
+          low_nonzero = min(low_nonzero, u - 1);
+        }
+        const uint32_t bit = 1u << (i * S + j);
+        if (top >= 0xff000000u) bad |= bit;
+        if constexpr (kForm == kPlain) continue;
+        if (low_nonzero < (uint32_t(127 - 110) << 24) - 1) bad |= bit;
+        if (low < uint32_t(127 - 64) << 24 && n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n) small |= bit;
+      }
     int tail = lane;
     asm("" : "+v"(tail));  // addresses made from it are not formed before the loop and kept through it
-    if (__any(small != 0) &&
+    if (kForm != kPlain && __any(small != 0) &&
         __any(TinyActivation<kForm>(p, m0 + wm * (BM / 2), BM / 2, c0, c0 + chunks, pad, tail)))
       bad |= small;
 #pragma unroll
@@ -562,15 +579,7 @@ __global__ void SplitAImageKernel(const float* __restrict__ a, uint32_t* __restr
   }
   uint32_t part[3][4];
 #pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    const float x0 = x[2 * h];
-    const float x1 = x[2 * h + 1];
-    part[0][h] = PackBf16(x0, x1);
-    const float r0 = x0 - Bf16Low(part[0][h]);
-    const float r1 = x1 - Bf16High(part[0][h]);
-    part[1][h] = PackBf16(r0, r1);
-    part[2][h] = PackBf16(r0 - Bf16Low(part[1][h]), r1 - Bf16High(part[1][h]));
-  }
+  for (int h = 0; h < 4; ++h) SplitBf16PairAny(x[2 * h], x[2 * h + 1], part[0][h], part[1][h], part[2][h]);
   uint32_t* dst = img + blk * kImgBlockWords + ImageWord<kSwz>(r, g);
 #pragma unroll
   for (int pl = 0; pl < 3; ++pl)
@@ -1131,7 +1140,7 @@ __global__ __launch_bounds__(kSmallThreads) void GemmQ8SmallKernel(const float* 
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
       uint32_t ph, pm, pl;
-      SplitBf16Pair(x[2 * h], x[2 * h + 1], ph, pm, pl);
+      SplitBf16PairAny(x[2 * h], x[2 * h + 1], ph, pm, pl);
       hi[h] = ph;
       mid[h] = pm;
       lo[h] = pl;

@@ -789,18 +789,18 @@ constexpr int kSplitGroupBytes = kSplitTiles * kNarrowTile;  // bytes of one row
 
 // One 32-row block of a lane: its four weight loads w (rows 8g + 2h, 8g + 2h + 1 of its tile
 // in load h) and its 8 activations x (rows 8g .. 8g + 7) into the 8 accumulators, hi, then
-// mid, then lo parts.
+// mid, then lo parts. kAny: activations that are not finite or above the largest bf16 too.
+template <bool kAny>
 __device__ __forceinline__ void SplitBf16Block(const u32x4 (&w)[4], const f32x2 (&x)[4], v4f (&acc)[kNarrowTile]) {
   u32x4 ah, am, al;
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
-    const float x0 = x[h][0];
-    const float x1 = x[h][1];
-    ah[h] = PackBf16(x0, x1);
-    const float r0 = x0 - Bf16Low(ah[h]);
-    const float r1 = x1 - Bf16High(ah[h]);
-    am[h] = PackBf16(r0, r1);
-    al[h] = PackBf16(r0 - Bf16Low(am[h]), r1 - Bf16High(am[h]));
+    uint32_t hi, mid, lo;
+    if constexpr (kAny) SplitBf16PairAny(x[h][0], x[h][1], hi, mid, lo);
+    else SplitBf16Pair(x[h][0], x[h][1], hi, mid, lo);
+    ah[h] = hi;
+    am[h] = mid;
+    al[h] = lo;
   }
   // Column c of the tile: row 8g + 2h in byte c of words 0..1 of load h, row 8g + 2h + 1 in
   // words 2..3.
@@ -970,13 +970,33 @@ __global__ __launch_bounds__(kSplitThreads) void GemvSplitBf16Kernel(const int8_
     for (int u = 0; u < kSplitBatch; ++u) load_block(j + u, w[u], x[u]);
     __builtin_amdgcn_sched_barrier(0);  // every load of the batch is issued before any is used
 #pragma unroll
-    for (int u = 0; u < kSplitBatch; ++u) SplitBf16Block(w[u], x[u], acc);
+    for (int u = 0; u < kSplitBatch; ++u) SplitBf16Block<false>(w[u], x[u], acc);
   }
   for (; j < nb; ++j) {
     u32x4 w[4];
     f32x2 x[4];
     load_block(j, w, x);
-    SplitBf16Block(w, x, acc);
+    SplitBf16Block<false>(w, x, acc);
+  }
+
+  // An infinity, a NaN or a value above the largest bf16 leaves sums that are not finite (and so their
+  // total): the wave takes its blocks again. (The split for any value in the loop: 4096 x 14336, m = 5
+  // 14.3 -> 14.9 us.)
+  float total = 0.f;
+#pragma unroll
+  for (int c = 0; c < kNarrowTile; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) total += acc[c][r];
+  if (__any(!(fabsf(total) < INFINITY))) {
+#pragma unroll
+    for (int c = 0; c < kNarrowTile; ++c) acc[c] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (j = 0; j < nb; ++j) {
+      u32x4 w[4];
+      f32x2 x[4];
+      load_block(j, w, x);
+      SplitBf16Block<true>(w, x, acc);
+    }
   }
 
   SplitBf16Finish<kPlain>(p, m, splits, partials, arrivals, acc, red, &is_last, group, split);

@@ -134,7 +134,9 @@ ACCEL_HIP_API int accel_hip_matmul(AccelHipBuffer a, AccelHipBuffer b, AccelHipB
  * that, an int8 weight with k >= 32 and n >= 8 runs on the bf16 matrix cores with the activation
  * split exactly into three bf16 parts (with a per-column or whole-tensor scale, no zero points,
  * k % 32 == 0 and n % 8 == 0 the weight is staged once as bf16); smaller ones on the fp32 MFMA
- * GEMM with the int8 panel dequantized in LDS. */
+ * GEMM with the int8 panel dequantized in LDS. Infinite and NaN activations come out as fp32 products
+ * of them do. Activations below 2^-110 keep their leading bits down to 2^-134 on the staged bf16 and
+ * group-interleaved copies and all of them elsewhere, where they show in the result. */
 ACCEL_HIP_API int accel_hip_matmul_quantized(const float* a, const AccelHipQuantPlane* a_quant, const float* b,
                                              const AccelHipQuantPlane* b_quant, float* c, int64_t m, int64_t k,
                                              int64_t n);

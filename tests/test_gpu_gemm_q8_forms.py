@@ -113,3 +113,32 @@ def test_gemm_q8_forms_activations_below_the_parts(m, k, n, mode, zero):
     up = np.float64(2.0 ** 43)  # exact: the bound's absolute term stays below what subnormal sums round
     assert_gamma_bound(got * up, a.astype(np.float64) * up, w)
     assert not got[68].any()
+
+
+# The plain form (128 and 64 tiles), the small kernel (k <= 768 and k = 1536), the image and wide
+# kernels, the group-interleaved GEMV and the in-place GEMV on the same kind of plane.
+PLAIN_SHAPES = [(333, 1024, 2048), (100, 2048, 1024), (40, 576, 192), (40, 1536, 256), (2100, 96, 2056), (700, 96, 6000),
+                (5, 4096, 8192), (16, 4096, 8192), (9, 1024, 512)]
+
+
+@pytest.mark.parametrize("m,k,n", PLAIN_SHAPES)
+def test_q8_plain_planes_not_finite_activations(m, k, n):
+    """Whole chunks, no zero points: rows with an infinity, a NaN and a value above the largest bf16
+    come out as fp32 products do, whichever kernel the size picks; the other rows are untouched."""
+    r = np.random.default_rng(5)
+    q, s, _ = weight(r, k, n, "col", False, unit_scale=True)
+    a = r.standard_normal((m, k)).astype(np.float32)
+    a[1, k - 1] = np.inf
+    a[2, 0] = np.nan
+    a[3] = 0
+    a[3, 50] = np.float32(-3.399e38)
+    q[50] = np.where(r.random(n) < 0.5, 1, 0)
+    q[k - 1, :8] = 0
+    print(f"q8 {m}x{k}x{n}", flush=True)
+    got = run(a, q, s, None, "col")
+    rest = [0] + list(range(4, m))
+    assert_gamma_bound(got[rest], a[rest], q)
+    same_bits(got[3], (a[3, 50] * q[50].astype(np.float32)) + np.float32(0))
+    last = q[k - 1].astype(np.float64)
+    same_bits(got[1], np.where(last > 0, np.inf, np.where(last < 0, -np.inf, np.nan)).astype(np.float32))
+    assert np.isnan(got[2]).all()
