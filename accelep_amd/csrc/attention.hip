@@ -976,9 +976,19 @@ int64_t CuCount() {
   return ctx.cu_count > 0 ? ctx.cu_count : 256;
 }
 
+}  // namespace
+
+// A workgroup of kFlashRows rows per CU leaves its partial sums.
+size_t AttentionFlashWorkBytes(int64_t head_dim) {
+  return static_cast<size_t>(kFlashRows * CuCount() * (2 + head_dim)) * sizeof(float);
+}
+
+namespace {
+
+// work / work_bytes: the caller's scratch, as LaunchAttention has it.
 void LaunchFlash(const float* q, const float* k, const float* v, float* out, int64_t seq, int64_t position,
                  int64_t heads, int64_t kv_heads, int64_t head_dim, hipStream_t stream, const int32_t* position_dev,
-                 int64_t top) {
+                 int64_t top, float* work, size_t work_bytes) {
   const int64_t blocks = (seq + kFlashRows - 1) / kFlashRows * heads;
   if (heads > 65535 || seq > 0x7fffffff || position > 0x7fffffff || kv_heads > 65535 || blocks > 0x7fffffff)
     Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention is too large");
@@ -986,10 +996,11 @@ void LaunchFlash(const float* q, const float* k, const float* v, float* out, int
   // A grid that leaves CUs idle over a long key range cuts the range, at least 128 keys each (the
   // combine costs about 3 us): 17 rows from position 500, 9 heads, 12.0 -> 9.5 us in four; 100 rows
   // from 1700, 4 heads of 128, 52 -> 16 us in eight; 300 rows from 0, 4 heads, 13.9 -> 14.4 in two.
+  // Where the partial sums have no room the range stays whole.
   int64_t splits = std::max<int64_t>(1, std::min<int64_t>(cus / blocks, (top + seq) / 128));
   const size_t bytes = static_cast<size_t>(seq * heads * splits * (2 + head_dim)) * sizeof(float);
-  if (splits > 1 && !ScratchReady(bytes, kTempFlags, 0)) splits = 1;
-  float* partial = splits > 1 ? static_cast<float*>(Workspace(bytes)) : nullptr;
+  if (splits > 1 && !(work != nullptr ? bytes <= work_bytes : ScratchReady(bytes, kTempFlags, 0))) splits = 1;
+  float* partial = splits == 1 ? nullptr : work != nullptr ? work : static_cast<float*>(Workspace(bytes));
   const dim3 grid(static_cast<uint32_t>(blocks * splits)), block(kFlashThreads);
 #define ACCEL_FLASH(D)                                                                                            \
   hipLaunchKernelGGL(AttentionFlashKernel<D>, grid, block, 0, stream, q, k, v, out, position_dev,                 \
@@ -1018,16 +1029,6 @@ void LaunchAttention(const float* q, const float* k, const float* v, float* out,
   // With a device position the scratch must fit the largest position it can hold.
   const int64_t top = position_dev != nullptr ? max_position : position;
   const int64_t rows = top + seq;
-  const size_t need = AttentionWorkBytes(seq, heads, top, head_dim);
-  float* scratch = nullptr;
-  if (need > 0) {
-    if (work != nullptr) {
-      if (work_bytes < need) Fail(ACCEL_HIP_INVALID_ARGUMENT, "attention scratch is too small");
-      scratch = work;
-    } else {
-      scratch = static_cast<float*>(Workspace(need));
-    }
-  }
   const bool aligned = (reinterpret_cast<uintptr_t>(k) % 16 == 0) && (reinterpret_cast<uintptr_t>(v) % 16 == 0) &&
                        head_dim % 4 == 0;
   const int vec = aligned ? static_cast<int>(head_dim) : 0;
@@ -1037,8 +1038,18 @@ void LaunchAttention(const float* q, const float* k, const float* v, float* out,
   const bool few = seq <= kSplitMaxSeq && rows >= 256 && blocks * ((rows + kChunk - 1) / kChunk) < 3 * CuCount();
   if (fast && seq > 1 && !few && (head_dim == 64 || head_dim == 128) && aligned && (reinterpret_cast<uintptr_t>(q) % 16 == 0) &&
       (reinterpret_cast<uintptr_t>(out) % 16 == 0)) {
-    LaunchFlash(q, k, v, out, seq, position, heads, kv_heads, head_dim, stream, position_dev, top);
+    LaunchFlash(q, k, v, out, seq, position, heads, kv_heads, head_dim, stream, position_dev, top, work, work_bytes);
     return;
+  }
+  const size_t need = AttentionWorkBytes(seq, heads, top, head_dim);
+  float* scratch = nullptr;
+  if (need > 0) {
+    if (work != nullptr) {
+      if (work_bytes < need) Fail(ACCEL_HIP_INVALID_ARGUMENT, "attention scratch is too small");
+      scratch = work;
+    } else {
+      scratch = static_cast<float*>(Workspace(need));
+    }
   }
   if (seq <= kSplitMaxSeq) {
     const int64_t chunks = (rows + kChunk - 1) / kChunk;

@@ -420,8 +420,9 @@ void LaunchRopeAppend(float* q, const float* k, const float* v, float* k_cache, 
 // state[0] += 1, state[1] += 1 (position and produced count of a decode loop).
 void LaunchAdvance(int32_t* state, hipStream_t stream);
 // max_position: with position_dev, the largest position the device word may hold. work /
-// work_bytes: caller-owned scratch (at least AttentionWorkBytes); null uses the library
-// workspace.
+// work_bytes: caller-owned scratch (at least AttentionWorkBytes, which the online-softmax kernel
+// does not need: it takes partial sums of at most AttentionFlashWorkBytes where they fit); null uses
+// the library workspace.
 // fast: several rows (seq > 1) with head_dim 64 or 128 may use the online-softmax kernel, whose sums
 // run in another order than the reference's (rounding only); otherwise the scores keep the
 // reference's bits.
@@ -455,6 +456,7 @@ int DecodeAttentionSplits(int64_t max_position);
 constexpr size_t kDecodeSplitMaxBytesPerHead = 64 * (2 + 64) * sizeof(float);
 // Scratch bytes LaunchAttention needs for these sizes (0 when none).
 size_t AttentionWorkBytes(int64_t seq, int64_t heads, int64_t max_position, int64_t head_dim);
+size_t AttentionFlashWorkBytes(int64_t head_dim);
 // rng_inout is a device word holding the xorshift32 state; index_dev offsets `chosen`.
 // greedy_work (at least GreedyWorkBytes(vocab) bytes, its first word zero and left zero by
 // each launch; launches sharing it must not overlap) lets a greedy pick run over many

@@ -21,6 +21,7 @@
 //    from a HIP graph, so a token costs its kernels' time and not ~450 host launches.
 // The tokenizer calls (src/llama_model.cc:183-205, :449-560) encode and decode on the host
 // with ByteBpe (tokenizer.cc) around the same Generate.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -856,9 +857,11 @@ ACCEL_LLAMA_API AccelLlama* accel_llama_create(const AccelLlamaConfig* config) {
     m->chosen = DevBuf(ctx * sizeof(int32_t));
     m->prompt_ids = DevBuf(ctx * sizeof(int32_t));
     m->words = DevBuf(64);
-    // Room for the chunk partials and for the fixed-split partials of the decode attention.
-    m->attn_work = DevBuf(std::max(AttentionWorkBytes(1, config->heads, config->context - 1, dim),
-                                   static_cast<size_t>(config->heads) * kDecodeSplitMaxBytesPerHead));
+    // Room for the chunk partials and for the fixed-split partials of the decode attention, and for
+    // the partial sums of a prompt's.
+    m->attn_work = DevBuf(std::max({AttentionWorkBytes(1, config->heads, config->context - 1, dim),
+                                    AttentionFlashWorkBytes(dim),
+                                    static_cast<size_t>(config->heads) * kDecodeSplitMaxBytesPerHead}));
     m->attn_arrivals = DevBuf(static_cast<size_t>(config->heads) * sizeof(uint32_t));
     m->greedy_work = DevBuf(GreedyWorkBytes(config->vocab));
     m->greedy_keys = DevBuf(static_cast<size_t>((config->vocab + 7) / 8) * sizeof(uint64_t));

@@ -2,6 +2,9 @@
 against the same causal softmax in float64: row blocks and key ranges whole and partial, one or
 several key ranges per row block, a key that only later rows see holding no finite value."""
 
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -63,3 +66,30 @@ def test_attention_flash_masked_values_are_not_read(position, value):
     others = np.arange(64) != 7
     np.testing.assert_allclose(got[9:, :, others], exact[9:, :, others], rtol=1e-5, atol=2e-6)
     assert not np.isfinite(got[9:, :, 7]).any()
+
+
+def test_attention_flash_takes_no_score_scratch():
+    """4096 rows from position 16384, 32 heads: the kernel that keeps scores in memory would take 10.7
+    GB for them. Only a few rows are compared (float64)."""
+    hip = C.CDLL(os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "lib", "libamdhip64.so"))
+
+    def free_bytes():
+        check(lib().accel_hip_synchronize())
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    seq, position, heads, dim = 4096, 16384, 32, 64
+    r = np.random.default_rng(3)
+    q = r.standard_normal((seq, heads, dim), dtype=np.float32)
+    k, v = (r.standard_normal((seq + position, 1, dim), dtype=np.float32) for _ in range(2))
+    out, scores = dev(np.zeros(q.shape, np.float32)), dev(np.zeros(len(k), np.float32))
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    before = free_bytes()
+    check(lib().accel_hip_attention(qd.buffer, kd.buffer, vd.buffer, scores.buffer, out.buffer, seq, position, heads, 1,
+                                    dim))
+    assert before - free_bytes() < 1 << 30
+    got = out.numpy()
+    for s in (0, 2049, seq - 1):
+        exact = want(q[s:s + 1, :2], k[:position + s + 1], v[:position + s + 1], position + s)
+        np.testing.assert_allclose(got[s, :2], exact[0], rtol=1e-5, atol=2e-6)
