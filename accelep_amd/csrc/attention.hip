@@ -990,8 +990,6 @@ void LaunchFlash(const float* q, const float* k, const float* v, float* out, int
                  int64_t heads, int64_t kv_heads, int64_t head_dim, hipStream_t stream, const int32_t* position_dev,
                  int64_t top, float* work, size_t work_bytes) {
   const int64_t blocks = (seq + kFlashRows - 1) / kFlashRows * heads;
-  if (heads > 65535 || seq > 0x7fffffff || position > 0x7fffffff || kv_heads > 65535 || blocks > 0x7fffffff)
-    Fail(ACCEL_HIP_INVALID_ARGUMENT, "Attention is too large");
   const int64_t cus = CuCount();
   // A grid that leaves CUs idle over a long key range cuts the range, at least 128 keys each (the
   // combine costs about 3 us): 17 rows from position 500, 9 heads, 12.0 -> 9.5 us in four; 100 rows
@@ -1036,7 +1034,8 @@ void LaunchAttention(const float* q, const float* k, const float* v, float* out,
   // (row, head, 64 positions) would come to several per CU (3 rows from position 8000, 32 heads:
   // 109 -> 36 us, 4 from 1775, 9 heads of 128: 17.5 -> 14.8; 2 from 1775, 9 heads: 9.2 -> 10.3).
   const bool few = seq <= kSplitMaxSeq && rows >= 256 && blocks * ((rows + kChunk - 1) / kChunk) < 3 * CuCount();
-  if (fast && seq > 1 && !few && (head_dim == 64 || head_dim == 128) && aligned && (reinterpret_cast<uintptr_t>(q) % 16 == 0) &&
+  const bool fits = position + seq <= 0x7fffffff;  // 32-bit positions in the kernel's arguments
+  if (fast && seq > 1 && !few && fits && (head_dim == 64 || head_dim == 128) && aligned && (reinterpret_cast<uintptr_t>(q) % 16 == 0) &&
       (reinterpret_cast<uintptr_t>(out) % 16 == 0)) {
     LaunchFlash(q, k, v, out, seq, position, heads, kv_heads, head_dim, stream, position_dev, top, work, work_bytes);
     return;

@@ -44,14 +44,19 @@ def inputs(seq, position, heads, kv_heads, dim):
 
 
 # (2, 0): fewer keys than one wave's step. (40, 700) and (5, 2100): the key range in several parts,
-# the last ones short. (300, 0, 64 heads): more workgroups than CUs.
+# the last ones short. (300, 0, 64 heads): more workgroups than CUs. 65537
+# heads: more than a grid's second dimension holds.
 @pytest.mark.parametrize("seq,position,heads,kv_heads,dim", [
     (2, 0, 3, 1, 64), (5, 0, 2, 2, 128), (16, 0, 4, 2, 64), (17, 3, 9, 3, 64), (33, 64, 3, 3, 128), (65, 1, 4, 1, 64),
-    (40, 700, 6, 2, 64), (5, 2100, 4, 4, 128), (300, 0, 64, 8, 64), (3, 131, 32, 8, 128)])
+    (40, 700, 6, 2, 64), (5, 2100, 4, 4, 128), (300, 0, 64, 8, 64), (3, 131, 32, 8, 128), (2, 1, 65537, 65537, 64)])
 def test_attention_flash_against_float64(seq, position, heads, kv_heads, dim):
     q, k, v = inputs(seq, position, heads, kv_heads, dim)
     print(f"attention {seq} rows from {position}, {heads}/{kv_heads} heads of {dim}", flush=True)
-    np.testing.assert_allclose(run(q, k, v, position), want(q, k, v, position), rtol=1e-5, atol=2e-6)
+    got = run(q, k, v, position)
+    if heads > 65535:  # the first and the last heads are enough of them
+        some = np.r_[0:20, heads - 20:heads]
+        got, q, k, v = got[:, some], q[:, some], k[:, some], v[:, some]
+    np.testing.assert_allclose(got, want(q, k, v, position), rtol=1e-5, atol=2e-6)
 
 
 @pytest.mark.parametrize("position", [0, 900])
