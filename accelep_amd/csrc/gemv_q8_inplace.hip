@@ -75,7 +75,7 @@ struct Q8InPlaceArgs {
   const float* scale;
   const int8_t* zero;
   int32_t mode;
-  int32_t const_index;
+  int64_t const_index;
   float* c;
   Epilogue epi;
 };
@@ -262,8 +262,11 @@ __device__ uint32_t TinyRows(const float* a, const Q8InPlaceArgs& p, int32_t m, 
   return tiny;
 }
 
-// What the first loads need leads the arguments (preloaded into SGPRs at wave launch). Grid: one
-// dimension, a multiple of 8 workgroups; those of one XCD (blockIdx.x % 8) take consecutive
+// Workgroups of a grid's first dimension at most: a dimension holds less than 2^32 threads.
+constexpr uint32_t kGridX = uint32_t(1) << 22;
+
+// What the first loads need leads the arguments (preloaded into SGPRs at wave launch). Grid: a
+// multiple of 8 workgroups; those of one XCD (blockIdx.x % 8) take consecutive
 // (column group, split) pairs, so the splits of a group meet in one L2. Up to V = 4 two workgroups
 // share a CU (at most 128 VGPRs; the compiler would take 132 to 152).
 template <int V, int kForm>
@@ -281,9 +284,10 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(V <
   const int slot = lane & 15;
   const int g = lane >> 4;
   if (tid == 0) again[0] = again[1] = 0;
-  const int per_xcd = static_cast<int>(gridDim.x / kXcds);
-  const int pair = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
-  if (pair >= pairs) return;
+  const uint32_t per_xcd = (static_cast<uint32_t>(pairs) + kXcds - 1) / kXcds;
+  const uint32_t b = blockIdx.y * kGridX + blockIdx.x;  // one row of workgroups, but for huge n
+  const int pair = static_cast<int>(b % kXcds * per_xcd + b / kXcds);
+  if (b / kXcds >= per_xcd || pair >= pairs) return;
   const int group = pair / splits;
   const int split = pair - group * splits;
   const int kb = split * rows_per_split;
@@ -445,13 +449,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(V <
 }
 
 template <int V>
-void LaunchForm(int form, uint32_t grid, hipStream_t stream, const int8_t* q, const float* a, float* partials,
+void LaunchForm(int form, dim3 grid, hipStream_t stream, const int8_t* q, const float* a, float* partials,
                 uint32_t* arrivals, int32_t m, int32_t k, int32_t rows, int32_t splits, int32_t pairs, int64_t n,
                 const Q8InPlaceArgs& args) {
   switch (form) {
 #define ACCEL_Q8_INPLACE(F)                                                                                      \
   case F:                                                                                                        \
-    hipLaunchKernelGGL((GemvQ8InPlaceKernel<V, F>), dim3(grid), dim3(64 * kWaves), 0, stream, q, a, partials, arrivals, \
+    hipLaunchKernelGGL((GemvQ8InPlaceKernel<V, F>), grid, dim3(64 * kWaves), 0, stream, q, a, partials, arrivals, \
                        m, k, rows, splits, pairs, n, args);                                                      \
     break;
     ACCEL_Q8_INPLACE(kNone) ACCEL_Q8_INPLACE(kZero) ACCEL_Q8_INPLACE(kRow) ACCEL_Q8_INPLACE(kRowZero)
@@ -465,8 +469,7 @@ void LaunchGemvQ8InPlace(const float* a, const Q8View& b, float* c, int64_t m, i
                          const Epilogue& epi, hipStream_t stream) {
   const Context& ctx = Ctx();
   const int64_t cus = ctx.cu_count > 0 ? ctx.cu_count : 256;
-  if (m < 1 || m > 16 || k < 1 || n < 1 || k >= (int64_t(1) << 28) || n >= (int64_t(1) << 34) ||
-      b.const_index > 0x7fffffff)
+  if (m < 1 || m > 16 || k < 1 || n < 1 || k >= (int64_t(1) << 28) || n >= (int64_t(1) << 34))
     Fail(ACCEL_HIP_INVALID_ARGUMENT, "GEMV too large");
   // Bytes of a row a lane reads. Long runs use whole cache lines, short ones give a small matrix
   // enough workgroups without a split of K (m = 16: 576 x 3072 4.8 us at 2, 5.5 at 4, 7.6 at 8;
@@ -495,7 +498,7 @@ void LaunchGemvQ8InPlace(const float* a, const Q8View& b, float* c, int64_t m, i
   args.scale = b.scale;
   args.zero = b.zero;
   args.mode = b.mode;
-  args.const_index = static_cast<int32_t>(b.const_index);
+  args.const_index = b.const_index;
   args.c = c;
   args.epi = epi;
   float* partials = nullptr;
@@ -504,7 +507,8 @@ void LaunchGemvQ8InPlace(const float* a, const Q8View& b, float* c, int64_t m, i
     partials = static_cast<float*>(Workspace(part_bytes(splits)));
     arrivals = static_cast<uint32_t*>(Temp(kTempArrivals, count_bytes));
   }
-  const uint32_t grid = static_cast<uint32_t>((pairs + kXcds - 1) / kXcds * kXcds);
+  const uint32_t blocks = static_cast<uint32_t>((pairs + kXcds - 1) / kXcds * kXcds);
+  const dim3 grid(std::min(blocks, kGridX), (blocks + kGridX - 1) / kGridX);
   const int form = b.mode == kScalePerRow ? (b.zero != nullptr ? kRowZero : kRow) : (b.zero != nullptr ? kZero : kNone);
   const int32_t m32 = static_cast<int32_t>(m), k32 = static_cast<int32_t>(k), rows32 = static_cast<int32_t>(rows);
   const int32_t splits32 = static_cast<int32_t>(splits), pairs32 = static_cast<int32_t>(pairs);

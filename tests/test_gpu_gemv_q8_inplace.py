@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from hip_helpers import Epilogue, assert_gamma_bound, check, dev, lib, quant_plane, same_bits
+from hip_helpers import DeviceArray, Epilogue, assert_gamma_bound, check, dev, lib, quant_plane, same_bits
 from test_gpu_gemm_q8_forms import FORMS, dequant, run, weight
 
 pytestmark = pytest.mark.gpu
@@ -116,3 +116,23 @@ def test_gemv_q8_in_place_in_a_capture(m, zero):
             assert_gamma_bound(cd.numpy(), a, dequant(q, s, z, "col"))
     finally:
         lib().accel_hip_graph_destroy(graph)
+
+
+def test_gemv_q8_in_place_more_columns_than_one_grid_dimension():
+    """2^30 and a few columns: more threads than one dimension of a grid holds. Integer products, so
+    the compared spans are exact: the ends, the last whole group and where the second row of workgroups
+    starts."""
+    m, k, n = 3, 1, (1 << 30) + 1043
+    r = np.random.default_rng(1)
+    q = np.frombuffer(r.bytes(n), np.int8)
+    qd, sd = dev(q), dev(np.ones(1, np.float32))
+    a = np.array([[1], [-2], [3]], np.float32)
+    ad, cd = dev(a), DeviceArray((m, n))
+    plane = quant_plane(qd, sd, None, [k, n], -1)
+    check(lib().accel_hip_matmul_quantized(ad.ptr, None, None, C.byref(plane), cd.ptr, m, k, n))
+    span = 2048
+    for row in range(m):
+        for start in (0, (1 << 29) - 1024, (1 << 29) + (1 << 27) - 1024, (1 << 30) - 1024, n - span):
+            got = np.empty(span, np.float32)
+            check(lib().accel_hip_peek(got.ctypes.data, cd.at(row * n + start), got.nbytes))
+            same_bits(got, a[row, 0] * q[start:start + span].astype(np.float32) + np.float32(0))
