@@ -1322,17 +1322,16 @@ struct Q8Plan {
   int64_t splits;
 };
 
-Q8Plan PlanQ8Gemm(int64_t m, int64_t n, int64_t chunks, int64_t cus) {
+Q8Plan PlanQ8Gemm(int64_t m, int64_t n, int64_t chunks, int64_t cus, int64_t max_splits) {
   constexpr double kChunk128[3] = {0, 1.0, 1.75};
   constexpr double kChunk64[4] = {0, 0.6, 0.8, 1.06};
-  constexpr int64_t kMaxSplits = 16;
   Q8Plan best{128, 1};
   double best_us = 0;
   for (const int bm : {128, 64}) {
     const int64_t tiles = ((m + bm - 1) / bm) * ((n + bm - 1) / bm);
     const int64_t cap = bm == 128 ? 2 : 3;
     const double* us = bm == 128 ? kChunk128 : kChunk64;
-    for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(kMaxSplits, chunks / 3)); ++s) {
+    for (int64_t s = 1; s <= std::max<int64_t>(1, std::min(max_splits, chunks / 3)); ++s) {
       if (s > 1 && tiles * (s - 1) >= cap * cus) break;  // the CUs are full with fewer splits
       const int64_t per_cu = (tiles * s + cus - 1) / cus;
       double t = ((per_cu / cap) * us[cap] + us[per_cu % cap]) * static_cast<double>((chunks + s - 1) / s);
@@ -1414,17 +1413,23 @@ bool LaunchGemmQ8Bf16(const float* a, const Q8View& b, float* c, int64_t m, int6
   Context& ctx0 = Ctx();
   const int64_t cus = ctx0.cu_count > 0 ? ctx0.cu_count : 256;
   const int64_t chunks = (k + kBK - 1) / kBK;
-  const Q8Plan plan = PlanQ8Gemm(m, n, chunks, cus);
+  // With a split K (ranges of whole chunks) a second kernel adds the partial sums in split order.
+  // Where the partial sums have no room (inside a capture, or the no-allocation scratch) the tiles are
+  // those of the best plan that keeps K whole.
+  constexpr int64_t kMaxSplits = 16;
+  Q8Plan plan = PlanQ8Gemm(m, n, chunks, cus, kMaxSplits);
+  int64_t cper = (chunks + plan.splits - 1) / plan.splits;
+  int64_t splits = (chunks + cper - 1) / cper;
+  if (splits > 1 && !ScratchReady(static_cast<size_t>(splits * m * n) * sizeof(float), kTempFlags, 0)) {
+    plan = PlanQ8Gemm(m, n, chunks, cus, 1);
+    splits = 1;
+    cper = chunks;
+  }
   const int bm = plan.bm;
   const int64_t tiles_m = (m + bm - 1) / bm;
   const int64_t tiles_n = (n + bm - 1) / bm;
   const int64_t tiles = tiles_m * tiles_n;
   if (tiles * kBand > 0x7fffffff) return false;
-  // With a split K (ranges of whole chunks) a second kernel adds the partial sums in split order.
-  // Where the partial sums have no room (inside a capture, or the no-allocation scratch) K stays whole.
-  const int64_t cper = (chunks + plan.splits - 1) / plan.splits;
-  int64_t splits = (chunks + cper - 1) / cper;
-  if (splits > 1 && !ScratchReady(static_cast<size_t>(splits * m * n) * sizeof(float), kTempFlags, 0)) splits = 1;
   Q8GemmArgs args;
   args.a = a;
   args.q = b.q;
@@ -1440,7 +1445,7 @@ bool LaunchGemmQ8Bf16(const float* a, const Q8View& b, float* c, int64_t m, int6
   args.tiles_n = static_cast<int32_t>(tiles_n);
   args.tiles = static_cast<int32_t>(tiles);
   args.tiles_per_xcd = static_cast<int32_t>((tiles + kXcds - 1) / kXcds);
-  args.chunks_per_split = splits > 1 ? cper : chunks;
+  args.chunks_per_split = cper;
   args.partials = nullptr;
   args.epi = epi;
   if (splits > 1) args.partials = static_cast<float*>(Workspace(static_cast<size_t>(splits * m * n) * sizeof(float)));

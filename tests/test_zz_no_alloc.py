@@ -123,3 +123,30 @@ def test_noalloc_refuses_scratch_beyond_its_size():
     assert rc == INVALID_ARGUMENT, (rc, msg)
     assert "no-allocation scratch" in msg
     assert (out.numpy() == 3.0).all()
+
+
+@pytest.mark.parametrize("quantized_b", [True, False])
+def test_noalloc_gemm_whose_partial_sums_have_no_room(quantized_b):
+    """A quantized A takes 48 MB of the scratch (dequantized), which leaves too little for the partial
+    sums of the K split that the allocating call makes: K stays whole and the product is right."""
+    L = lib()
+    m, k, n = 1000, 12001, 1024
+    r = np.random.default_rng(4)
+    qa, sa = r.integers(-127, 128, size=m * k, dtype=np.int8), r.uniform(1e-3, 1e-2, m).astype(np.float32)
+    qad, sad = dev(qa), dev(sa)
+    aq = quant_plane(qad, sad, None, [m, k], 0)
+    a = qa.reshape(m, k).astype(np.float32) * sa[:, None]
+    out = dev(np.full((m, n), 3.0, np.float32))
+    if quantized_b:
+        qb, sb = r.integers(-127, 128, size=k * n, dtype=np.int8), r.uniform(1e-3, 1e-2, n).astype(np.float32)
+        qbd, sbd = dev(qb), dev(sb)
+        bq = quant_plane(qbd, sbd, None, [k, n], 1)
+        w = qb.reshape(k, n).astype(np.float32) * sb
+        args = (None, C.byref(aq), None, C.byref(bq))
+    else:
+        w = r.standard_normal((k, n)).astype(np.float32)
+        bd = dev(w)
+        args = (None, C.byref(aq), bd.ptr, None)
+    for fn in (L.accel_hip_matmul_quantized_fused_noalloc, L.accel_hip_matmul_quantized_fused):
+        check(fn(*args, out.ptr, m, k, n, None))
+        assert_gamma_bound(out.numpy(), a, w)
