@@ -26,9 +26,9 @@
 //    the loss it can reach larger sums; without one, a sum of 2^-64 or more loses at most k 2^-102,
 //    k 2^-38 of it). There the workgroup reads its operands again, and the tile is summed again if one
 //    of them is not zero and below 2^-110. 1000 x 4096 x 4096: following the largest operand takes 1.4
-//    us (187 us with the lowest exponent followed too), the second reading 27 us, one infinity in A 104,
-//    a row of 1e-37 204 (349 us in all on the fp32 matrix cores alone; 64 x 64 tiles summed again one k
-//    pair after the other: 440 and 620).
+//    to 4 us (2 % on the slower of two cards; 9 us more with the lowest exponent followed too), the
+//    second reading 30 us, one infinity in A 130, a row of 1e-37 200 (349 us in all on the fp32 matrix
+//    cores alone; 64 x 64 tiles summed again one k pair after the other: 440 and 620).
 #include "device_common.h"
 
 #include <algorithm>
@@ -85,6 +85,8 @@ __device__ __forceinline__ void LoadRaw(const float* a, const float* b, int64_t 
 
 // Operands of this size and more may lift what the parts lose of a tiny one over 2^-64.
 constexpr float kHuge = 0x1p32f;
+// A workgroup met such an operand; it has a sum below 2^-64 (zero too).
+constexpr uint32_t kSeenHuge = 1, kSeenSmall = 2;
 
 // largest = max(largest, |x0|, |x1|) in one instruction (NaNs, which the sums show, are left out).
 __device__ __forceinline__ void KeepLargest(float& largest, float x0, float x1) {
@@ -193,6 +195,7 @@ GemmF32PartsKernel(PartsArgs p) {
   constexpr int S = Shape<BM>::kS;
   constexpr int kGroups = Shape<BM>::kGroups;
   __shared__ u32x4 lds[2 * Shape<BM>::kBufVecs];
+  __shared__ uint32_t seen;  // kSeenHuge, kSeenSmall: over the workgroup
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -243,6 +246,7 @@ GemmF32PartsKernel(PartsArgs p) {
     for (int e = 0; e < 8; ++e)
       if (8 * ag + e >= kBK - pad) raw[0].a[e >> 2][e & 3] = 0.f;
   }
+  if (tid == 0) seen = 0;
   float largest = 0.f;  // of the operands this thread splits, without the sign
   StoreRaw<BM>(lds, a_piece, b_piece, raw[0], largest);
   __syncthreads();
@@ -276,35 +280,39 @@ GemmF32PartsKernel(PartsArgs p) {
     }
   }
 
-  // Of a tile's sums in this lane: not finite, or not zero and below 2^-110; zero or below 2^-64.
-  bool bad[S][S], small[S][S], any_small = false;
+  uint32_t top = 0, low = 0xffffffffu;  // of the sums' bits without the sign
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < S; ++j) {
-      uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
+    for (int j = 0; j < S; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         hh[i][j][r] = hh[i][j][r] + cross[i][j][r];
         const uint32_t u = __float_as_uint(hh[i][j][r]) << 1;
         top = max(top, u);
         low = min(low, u);
-        low_nonzero = min(low_nonzero, u - 1);
       }
-      bad[i][j] = top >= 0xff000000u || low_nonzero < (uint32_t(127 - 110) << 24) - 1;
-      small[i][j] = low < uint32_t(127 - 64) << 24;
-      any_small |= small[i][j];
-    }
-  const bool huge = __syncthreads_or(largest >= kHuge);
-  bool tiny = false;
-  if (__syncthreads_or(huge || any_small))
-    tiny = __syncthreads_or(TinyOperand(asrc, bsrc, p.n, c0, c0 + chunks, pad));
+  constexpr uint32_t kInf = 0xff000000u, k2m64 = uint32_t(127 - 64) << 24, k2m110 = uint32_t(127 - 110) << 24;
+  const uint32_t look = (__any(largest >= kHuge) ? kSeenHuge : 0u) | (__any(low < k2m64) ? kSeenSmall : 0u);
+  if (lane == 0 && look != 0) atomicOr(&seen, look);
+  __syncthreads();
+  const bool huge = (seen & kSeenHuge) != 0;
+  const bool tiny = seen != 0 && __syncthreads_or(TinyOperand(asrc, bsrc, p.n, c0, c0 + chunks, pad));
+  if (__any(top >= kInf || low < k2m64) || (tiny && huge)) {
 #pragma unroll
-  for (int i = 0; i < S; ++i)
+    for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < S; ++j)
-      if (__any(bad[i][j] || (tiny && (huge || small[i][j]))))
-        PlainSums<BM>(p, m0 + (wm * S + i) * 32, n0 + (wn * S + j) * 32, c0, c0 + chunks, pad, lane, kg, hh[i][j]);
+      for (int j = 0; j < S; ++j) {
+        bool again = tiny && huge;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t u = __float_as_uint(hh[i][j][r]) << 1;
+          again |= u >= kInf || u - 1 < k2m110 - 1 || (tiny && u < k2m64);
+        }
+        if (__any(again))
+          PlainSums<BM>(p, m0 + (wm * S + i) * 32, n0 + (wn * S + j) * 32, c0, c0 + chunks, pad, lane, kg, hh[i][j]);
+      }
+  }
 
   // Two waves hold a 64 x 64 tile's sums over the two halves of each chunk: wave kg finishes column
   // tile kg and gives its sums of the other one away through LDS.

@@ -450,34 +450,36 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
   // its K ranges can be short (333 x 1024 x 2048 19.8 us, 21.1 with every sum looked at).
   uint32_t bad = 0, small = 0;
   float total = 0.f;
+  uint32_t top = 0, low = 0xffffffffu;  // of the bits without the sign
 #pragma unroll
   for (int i = 0; i < S; ++i)
 #pragma unroll
-    for (int j = 0; j < S; ++j) {
+    for (int j = 0; j < S; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
-        if constexpr (kForm == kPlain) total += acc[i][j][r];
+        if constexpr (kForm == kPlain) {
+          total += acc[i][j][r];
+        } else {
+          const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
+          top = max(top, u);
+          low = min(low, u);
+        }
       }
-    }
-  if (kForm != kPlain || __any(!(fabsf(total) < INFINITY))) {
+  constexpr uint32_t kInf = 0xff000000u, k2m64 = uint32_t(127 - 64) << 24, k2m110 = uint32_t(127 - 110) << 24;
+  if (__any(kForm == kPlain ? !(fabsf(total) < INFINITY) : top >= kInf || low < k2m64)) {
 #pragma unroll
     for (int i = 0; i < S; ++i)
 #pragma unroll
       for (int j = 0; j < S; ++j) {
-        uint32_t top = 0, low = 0xffffffffu, low_nonzero = 0xffffffffu;  // of the bits without the sign
+        const bool live = n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
-          top = max(top, u);
-          low = min(low, u);
-          low_nonzero = min(low_nonzero, u - 1);
+          const uint32_t bit = 1u << (i * S + j);
+          if (u >= kInf || (kForm != kPlain && u - 1 < k2m110 - 1)) bad |= bit;
+          if (kForm != kPlain && live && u < k2m64) small |= bit;
         }
-        const uint32_t bit = 1u << (i * S + j);
-        if (top >= 0xff000000u) bad |= bit;
-        if constexpr (kForm == kPlain) continue;
-        if (low_nonzero < (uint32_t(127 - 110) << 24) - 1) bad |= bit;
-        if (low < uint32_t(127 - 64) << 24 && n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n) small |= bit;
       }
     int tail = lane;
     asm("" : "+v"(tail));  // addresses made from it are not formed before the loop and kept through it
