@@ -1,8 +1,9 @@
 """The cross-workgroup hand-overs of the built library, checked in its gfx950 machine code.
 
-Three kernels add other workgroups' results inside one launch:
-* GemvSplitBf16Kernel (the K splits of a column group) and DecodeAttentionKernel (the chunks
-  of a head) store their partial results with agent-scope relaxed atomic stores
+Five kernels add other workgroups' results inside one launch:
+* GemvSplitBf16Kernel, GemvQ8InPlaceKernel and GemvF32Kernel (the K splits of a column group) and
+  DecodeAttentionKernel (the chunks of a head) store their partial results with agent-scope relaxed
+  atomic stores
   (`global_store ... sc1`, written through to the level every XCD reads), bump an arrival
   counter with an agent-scope atomic add, and the workgroup that completes the count reads
   the partials with agent-scope relaxed atomic loads (`global_load ... sc1`);
@@ -44,6 +45,11 @@ KERNELS = [
     ("GemvSplitBf16KernelILb0EE", True, False),
     ("21DecodeAttentionKernel", True, False),
     ("12GreedyKernel", False, True),
+    # columns a lane, plane form
+    *[(f"19GemvQ8InPlaceKernelILi{v}ELi{form}EE", True, False) for v in (1, 2, 4, 8) for form in range(4)],
+    # columns a lane and rows a batch, streaming loads, input transform
+    *[(f"13GemvF32KernelILi{v}ELi8ELi{u}ELb{stream}ELi{form}EE", True, False)
+      for v, u in ((1, 8), (2, 4), (4, 4)) for stream in (0, 1) for form in range(3)],
 ]
 
 
