@@ -135,7 +135,7 @@ void RunMatmul(const float* a, const AccelHipQuantPlane* aq, const float* b, con
     } else if (q8 && m <= 16) {
       if (GemvWantsGroups(m, k, n, view)) view.grouped = StagedGroupTiles(view.q, k, n, ctx.stream, stage_weights);
       else if (GemvWantsTiles(m, k, n, view)) {
-        const bool in_place = Capturing() && GemvTilesOptional(m, k, n, view);
+        const bool in_place = GemvTilesOptional(m, k, n, view) && Capturing();
         view.tiled = StagedColumnTiles(view.q, k, n, ctx.stream, stage_weights && !in_place);
       }
       LaunchGemvQ8(a_f, view, c, m, k, n, main, ctx.stream);
