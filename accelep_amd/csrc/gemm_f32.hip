@@ -751,8 +751,10 @@ bool LaunchGemmF32(const float* a, const float* b, const Q8View& bq, float* c, i
     // 64 x 1536 x 576 20.4 us here, 11.3 there; 256 x 512 x 2048, half of the CUs, 11.0 and 13.0; the
     // MLP's 256 x 1024 x 4096 16.9 and 26.6). A round of 128 tiles is faster there too (1024 x 4096 x
     // 4096 206 us, 173 there), but its K chains are twice as long: error 1.9e-7 here, 2.7e-7 there. K
-    // ranges of exactly 1024 (the unrolled form) stay here at any grid (128 x 1024 x 1024 14.3 us,
-    // 11.1 there): a caller may count on their weight's staged parts.
+    // ranges of exactly 1024 (the unrolled form) stay here at any grid although they would be faster
+    // there too (128 x 1024 x 1024 14.3 us, 11.1 there): a graph captured on such a weight after its
+    // second use reads the staged parts, and is refused once the weight is rewritten. Programs and the
+    // capture tests rely on that refusal at these sizes; GemmF32PartsKernel would read the new values.
     const bool keep = 2 * wtiles * wsplits >= cus || k == wsplits * 4 * unit;
     if (k % (wsplits * unit) == 0 && keep && wtiles <= 0x7fffffff && m <= 0x7fffffff && n <= 0x7fffffff && k <= 0x7fffffff) {
       WsArgs ws;

@@ -123,7 +123,10 @@ ACCEL_HIP_API void accel_hip_reset_packed_probes(void);
 
 /* ---- compute ---------------------------------------------------------------------------- */
 /* Device::MatMul (include/accel/device.h:81-82; src/sim_device.cc:185-196): row-major
- * C[m, n] = A[m, k] @ B[k, n], overwrites C (zeros when k == 0). fp32 MFMA. */
+ * C[m, n] = A[m, k] @ B[k, n], overwrites C (zeros when k == 0). m <= 16 and k < 32: fp32 MFMA;
+ * otherwise six products of exact bf16 parts with fp32 results, summed again on the fp32 MFMA where the
+ * parts cannot hold the operands (except on small grids of whole 64 x 64 tiles, where operands below
+ * 2^-110 keep their bits down to 2^-134 and an infinity gives NaN). */
 ACCEL_HIP_API int accel_hip_matmul(AccelHipBuffer a, AccelHipBuffer b, AccelHipBuffer c, int64_t m, int64_t k,
                                    int64_t n);
 /* accel::MatMulQuantized (include/accel/runtime.h:124-125; src/sim_device.cc:541-602).
@@ -135,8 +138,9 @@ ACCEL_HIP_API int accel_hip_matmul(AccelHipBuffer a, AccelHipBuffer b, AccelHipB
  * split exactly into three bf16 parts (with a per-column or whole-tensor scale, no zero points,
  * k % 32 == 0 and n % 8 == 0 the weight is staged once as bf16); smaller ones on the fp32 MFMA
  * GEMM with the int8 panel dequantized in LDS. Infinite and NaN activations come out as fp32 products
- * of them do. Activations below 2^-110 keep their leading bits down to 2^-134 on the staged bf16 and
- * group-interleaved copies and all of them elsewhere, where they show in the result. */
+ * of them do. Activations below 2^-110 keep their bits down to 2^-134 on the group-interleaved copy
+ * and, above 16 rows, with the planes that are staged as bf16; elsewhere, where their lower bits show in
+ * the result, they keep all of them. */
 ACCEL_HIP_API int accel_hip_matmul_quantized(const float* a, const AccelHipQuantPlane* a_quant, const float* b,
                                              const AccelHipQuantPlane* b_quant, float* c, int64_t m, int64_t k,
                                              int64_t n);
@@ -145,10 +149,12 @@ ACCEL_HIP_API int accel_hip_matmul_quantized(const float* a, const AccelHipQuant
  * binds the weight (UploadDequantized and BindConstant, src/ep.cc:843-900,1430-1463). Builds
  * now, on the library stream, the staged copies of the int8 weight b_quant ([k, n] at its
  * offset) that the matmuls otherwise build at the weight's first use: layouts is a mask of
- * ACCEL_HIP_STAGE_*, 0 for every layout this plane's form allows. A copy lasts until the
- * weight's allocation is freed or written. Refused (ACCEL_HIP_RUNTIME_ERROR) during a graph
- * capture; ACCEL_HIP_INVALID_ARGUMENT for a layout the plane cannot take or a weight outside
- * this library's heap. *staged (if not NULL) receives the layouts built. */
+ * ACCEL_HIP_STAGE_*, 0 for every layout this plane's form allows, also one that no kernel reads
+ * at its size (the group-interleaved copy, k * n bytes, below 28 Mi weights: a mask leaves it out).
+ * A copy lasts until the weight's allocation is freed or written. Refused
+ * (ACCEL_HIP_RUNTIME_ERROR) during a graph capture; ACCEL_HIP_INVALID_ARGUMENT for a layout the
+ * plane cannot take or a weight outside this library's heap. *staged (if not NULL) receives the
+ * layouts built. */
 #define ACCEL_HIP_STAGE_GEMV_TILES 1u  /* 8-column tiles: the int8 GEMV at m <= 2, and at m <= 4 for small matrices */
 #define ACCEL_HIP_STAGE_GEMV_GROUPS 2u /* group-interleaved tiles: the bf16-split GEMV, 3 <= m <= 16, from 28 Mi weights */
 #define ACCEL_HIP_STAGE_GEMM_BF16 4u   /* bf16 in MFMA operand order: the int8-weight GEMM, m > 16 */
