@@ -452,9 +452,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
   float total = 0.f;
   uint32_t top = 0, low = 0xffffffffu;  // of the bits without the sign
 #pragma unroll
-  for (int i = 0; i < S; ++i)
+  for (int j = 0; j < S; ++j) {
+    uint32_t low_j = 0xffffffffu;
 #pragma unroll
-    for (int j = 0; j < S; ++j)
+    for (int i = 0; i < S; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         acc[i][j][r] = acc[i][j][r] + acc_ml[i][j][r];
@@ -463,9 +464,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BM == 
         } else {
           const uint32_t u = __float_as_uint(acc[i][j][r]) << 1;
           top = max(top, u);
-          low = min(low, u);
+          low_j = min(low_j, u);
         }
       }
+    if (n0 + wn * (BM / 2) + j * 32 + (lane & 31) < p.n) low = min(low, low_j);
+  }
   constexpr uint32_t kInf = 0xff000000u, k2m64 = uint32_t(127 - 64) << 24, k2m110 = uint32_t(127 - 110) << 24;
   if (__any(kForm == kPlain ? !(fabsf(total) < INFINITY) : top >= kInf || low < k2m64)) {
 #pragma unroll
